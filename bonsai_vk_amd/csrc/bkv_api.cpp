@@ -84,16 +84,34 @@ PrefillPlan plan_prefill(int nh, int nkv, uint32_t pos0, int n_q, size_t base) {
   return p;
 }
 
-// the exact prefill's workspace for chunks ending at or before max_ctx: per workgroup of one slice,
-// the [keys][rows] score / exp scratch; then (q8_0 V) the slice's sums and the PV kernel's partials
-static size_t prefill_exact_extra(int nh, int nkv) {
-  const size_t wgs = (size_t)nkv * (kPxSlice / kPxQ);
-  return align256(wgs * kPxRows * sizeof(float)) + align256((size_t)kPvSplit * kPxSlice * nh * kHd * sizeof(float));
+// The exact prefill runs a chunk in slices of queries, whose scores it keeps: at least kPxSlice
+// queries, more where their scores take at most kPxScratch (short contexts: fewer, fuller launches).
+struct PxLayout {
+  int64_t ld;                              // keys per query in the scratch (+ the exp sweep's overhang)
+  size_t sums, part, total;
+};
+static PxLayout px_layout(int nh, int nkv, int64_t max_ctx, int64_t slice, size_t base) {
+  PxLayout l;
+  l.ld = cdiv(max_ctx, kPxTile16) * kPxTile16 + kPxTile16;
+  const size_t units = (size_t)nkv * cdiv(slice, kPxQ);
+  l.sums = base + align256(units * (size_t)l.ld * kPxRows * sizeof(float));
+  l.part = l.sums + align256(units * kPxRows * sizeof(float));
+  l.total = l.part + align256((size_t)kPvSplit * kPxSlice * nh * kHd * sizeof(float));
+  return l;
 }
+static int64_t px_slice(int nkv, int64_t max_ctx, int64_t n_q) {
+  const int64_t ld = cdiv(max_ctx, kPxTile16) * kPxTile16 + kPxTile16;
+  const int64_t fit = (int64_t)(kPxScratch / ((size_t)nkv * ld * kGqa * sizeof(float))) / kPxQ * kPxQ;
+  return std::min<int64_t>(n_q, std::max<int64_t>(kPxSlice, std::min<int64_t>(fit, BKV_PREFILL_MAX_Q)));
+}
+// the workspace for chunks ending at or before max_ctx: the largest any of them asks for
 size_t prefill_exact_workspace(int nh, int nkv, int64_t max_ctx, size_t base) {
-  const int64_t ld = cdiv(max_ctx, kPxTile) * kPxTile + kPxTile;   // + the exp sweep's overhang
-  const size_t wgs = (size_t)nkv * (kPxSlice / kPxQ);
-  return base + align256(wgs * (size_t)ld * kPxRows * sizeof(float)) + prefill_exact_extra(nh, nkv);
+  const size_t least = px_layout(nh, nkv, max_ctx, kPxSlice, base).total;
+  const int64_t most = std::min<int64_t>(max_ctx, BKV_PREFILL_MAX_Q);
+  if (most <= kPxSlice) return least;
+  const size_t scratch = std::min<size_t>(kPxScratch, px_layout(nh, nkv, max_ctx, most, 0).sums);
+  return std::max(least, base + align256(scratch) + px_layout(nh, nkv, 1, BKV_PREFILL_MAX_Q, 0).total -
+                             px_layout(nh, nkv, 1, BKV_PREFILL_MAX_Q, 0).sums);
 }
 
 // the largest plan_prefill(...).total over every chunk length and start position
@@ -477,9 +495,13 @@ static int prefill_common(const bkv_cache_desc *d, int layer, uint32_t pos0, int
   if (((uintptr_t)workspace & 255u) != 0) return BKV_EALIGN;
   const size_t base = prefill_base(d);
   if (!prefill_mfma_requested() && n_q >= kPxMinQ) {
-    // the exact kernel, in slices of at most kPxSlice queries
-    const int64_t ld = cdiv((int64_t)pos0 + n_q, kPxTile) * kPxTile + kPxTile;
-    if (ws_bytes < prefill_exact_workspace(d->nh, d->nkv, (int64_t)pos0 + n_q, base)) return BKV_EWORKSPACE;
+    // the exact kernels, in equal slices (of kPxSlice queries in a workspace without room for more)
+    const int64_t ctx = (int64_t)pos0 + n_q;
+    if (ws_bytes < px_layout(d->nh, d->nkv, ctx, kPxSlice, base).total) return BKV_EWORKSPACE;
+    int64_t slice = px_slice(d->nkv, ctx, n_q);
+    if (ws_bytes < px_layout(d->nh, d->nkv, ctx, slice, base).total) slice = kPxSlice;
+    slice = cdiv(cdiv(n_q, cdiv(n_q, slice)), kPxQ) * kPxQ;
+    const PxLayout l = px_layout(d->nh, d->nkv, ctx, slice, base);
     char *w = (char *)workspace;
     PrefillXArgs a{};
     a.L = view(d, layer);
@@ -488,25 +510,19 @@ static int prefill_common(const bkv_cache_desc *d, int layer, uint32_t pos0, int
     a.pos0 = pos0;
     a.chunk_q = n_q;
     a.scale = d->scale;
-    a.ld = ld;
+    a.ld = l.ld;
     a.q = q;
     a.qs = qs;
     a.gs = gs;
     a.sc = (float *)(w + base);
-    {
-      const size_t scb = align256((size_t)d->nkv * (kPxSlice / kPxQ) * (size_t)ld * kPxRows * sizeof(float));
-      a.sums = (float *)(w + base + scb);
-      a.part = (float *)(w + base + scb + align256((size_t)d->nkv * (kPxSlice / kPxQ) * kPxRows * sizeof(float)));
-    }
+    a.sums = (float *)(w + l.sums);
+    a.part = a.mx = (float *)(w + l.part);
     a.gate = gate;
     a.out = out;
     a.out_gated = out_gated;
-#ifdef BKV_EXPERIMENT_TS
-    a.ts = (unsigned *)w + 32768;
-#endif
-    for (int qb = 0; qb < n_q; qb += kPxSlice) {
+    for (int qb = 0; qb < n_q; qb += (int)slice) {
       a.q_base = qb;
-      a.n_q = std::min(kPxSlice, n_q - qb);
+      a.n_q = std::min((int)slice, n_q - qb);
       a.nqb = (int)cdiv(a.n_q, kPxQ);
       if ((rc = hip_fail(launch_prefill_exact(a, d->k_fmt, d->v_fmt, stream)))) return rc;
     }

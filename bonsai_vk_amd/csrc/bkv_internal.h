@@ -159,12 +159,14 @@ size_t prefill_workspace_bound(int nh, int nkv, size_t base);
 hipError_t launch_prefill(const PrefillArgs &a, int kf, int vf, hipStream_t st);
 
 // ------------------------------------------------------------------ exact chunked prefill
-constexpr int kPxQ = 4;          // queries per workgroup (x 4 heads = 16 rows)
+constexpr int kPxQ = 4;          // queries per unit (x 4 heads = 16 rows)
 constexpr int kPxRows = kPxQ * kGqa;
-constexpr int kPxTile = 256;     // keys per score / exp tile (one per lane of the workgroup)
-constexpr int kPxSlice = 512;    // queries per launch (bounds the score scratch)
-constexpr int kPvQ = 32;         // exact prefill, q8_0 V: queries per PV workgroup (4 kPvQ rows)
-constexpr int kPvSplit = 4;      // ... and key ranges per query block (partials added in order)
+constexpr int kPxTile = 64;      // keys per score tile, q8_0 K
+constexpr int kPxTile16 = 256;   // keys per score tile, fp16 K (and the scratch's granularity)
+constexpr int kPxSlice = 512;    // queries per launch, at least (the score scratch holds them)
+constexpr size_t kPxScratch = size_t(128) << 20;   // more queries per launch while their scores fit this
+constexpr int kPvQ = 32;         // queries per PV workgroup (4 kPvQ rows)
+constexpr int kPvSplit = 4;      // PV key ranges a slice of kPxSlice queries may have (shorter: more)
 constexpr int kPxMinQ = 16;      // shorter chunks run as decode rows
 
 struct PrefillXArgs {
@@ -174,19 +176,22 @@ struct PrefillXArgs {
   int q_base, n_q;               // this slice: queries q_base .. q_base + n_q - 1 of the chunk
   int chunk_q;                   // queries in the whole chunk (row stride of q / out)
   float scale;
-  int nqb;
-  int64_t ld;                    // keys per workgroup scratch region (multiple of kPxTile, one
-                                 // tile past the last key)
+  int nqb;                       // units (4 queries) of the slice
+  int ksplit, pv_split;          // key ranges of the score and PV kernels (set by the launcher)
+  int64_t ld;                    // keys per unit's scratch region (whole 256-key tiles, one more
+                                 // than its keys take)
   const float *q;                // [chunk_q][nh] rows of hd fp32, qs floats apart
   const float *gate;             // rows gs floats apart
   int qs, gs;
   float *out, *out_gated;
-  float *sc;                     // [nkv * nqb][ld][kPxRows] scores, then exp (the slice's workgroups)
-  float *sums;                   // q8_0 V: [nkv * nqb][kPxRows] the exact serial sums, for the PV kernel
-  float *part;                   // q8_0 V: [kPvSplit][kPxSlice][nh][hd] the PV kernel's key-range partials
-  unsigned *ts;                  // sweep timestamps (experiment builds), or null
+  float *sc;                     // [nkv * nqb][kPxQ][ld][kGqa] scores, then exp (the slice's units)
+  float *sums;                   // [nkv * nqb][kPxRows] the exact serial sums, for the PV kernel
+  float *part;                   // [pv_split][n_q][nh][hd] the PV kernel's key-range partials
+                                 // (pv_split * n_q <= kPvSplit * kPxSlice)
+  float *mx;                     // [nkv * nqb][ksplit][kPxRows] row maxima of the score kernel's key
+                                 // ranges (read before part, whose space they share, is written)
 };
-hipError_t launch_prefill_exact(const PrefillXArgs &a, int kf, int vf, hipStream_t st);
+hipError_t launch_prefill_exact(PrefillXArgs a, int kf, int vf, hipStream_t st);
 size_t prefill_exact_workspace(int nh, int nkv, int64_t max_ctx, size_t base);
 
 // ------------------------------------------------------------------ QK norm + rope + append

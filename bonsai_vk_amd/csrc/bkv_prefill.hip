@@ -23,6 +23,8 @@
 // What differs from the serial reference is only the order of the fp32 sums (dot products, the
 // softmax sum and PV), hence a tolerance rather than bit-exact parity for prefill.
 
+#include <type_traits>
+
 #include "bkv_device.h"
 #include "bkv_exp.h"
 #include "bkv_internal.h"
@@ -33,6 +35,8 @@ namespace bkv {
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef short v4s_t __attribute__((ext_vector_type(4)));
+typedef short v8s_t __attribute__((ext_vector_type(8)));
 
 constexpr int kPfNT = 256;      // 4 waves
 constexpr int kPfRS = 144;      // LDS row stride in bytes of the P and V^T tiles (64 fp16 + pad)
@@ -492,26 +496,20 @@ hipError_t launch_prefill(const PrefillArgs &a, int kf, int vf, hipStream_t st) 
 
 // ================================================================== exact prefill
 // The default prefill: every (query, head) row reproduces the serial reference bit for bit up to
-// the PV contraction. A workgroup owns 4 queries x 4 heads = 16 rows of one KV group and all of
-// their keys, in up to three sweeps:
-//   1  scores (q8_0 K: the correctly rounded inner sum of each block from the int8 matrix cores,
-//      bkv_q8dot.h, then acc = acc + f16(scale)*inner in block order; fp16 K: the reference's serial
-//      chain acc = acc + q16*k in ascending d, one exact fma per step on the fp32 matrix cores),
-//      times the softmax scale, masked causally; the row max. Scores go to a scratch region
-//      [key][row].
-//   2  e = exp(v - max) correctly rounded, written back over the scores; one lane per row adds
-//      them in key order (the reference's serial fp32 sum, attn_vk.h:175-189).
-//   3  (fp16 V) p16 = f16(e / sum) (the correctly rounded fp32 quotient, from e * (1/sum) by two
-//      remainder corrections, then round to nearest even), and out = sum p16 * v on the matrix
-//      cores. q8_0 V: the sums go out instead, and prefill_pv64_kernel forms p16 and the PV for 64
-//      rows at a time.
+// the PV contraction. A unit is 4 queries x 4 heads = 16 rows of one KV group; its scores live in a
+// scratch region [query][key][4 heads]. Four launches per slice of queries:
+//   scores  (q8_0 K: the correctly rounded inner sum of each block, bkv_q8dot.h's contract, then
+//           acc = acc + f16(scale)*inner in block order; fp16 K: the reference's serial chain
+//           acc = acc + q16*k in ascending d, one exact fma per step on the fp32 matrix cores),
+//           times the softmax scale, masked causally; the row maxima. The keys of a unit are split
+//           over workgroups so that short chunks fill the chip too.
+//   sums    e = exp(v - max) correctly rounded, written back over the scores; one lane per row adds
+//           them in key order (the reference's serial fp32 sum, attn_vk.h:175-189).
+//   pv      p16 = f16(e / sum) (the correctly rounded fp32 quotient, from e * (1/sum) by two remainder
+//           corrections, then round to nearest even), and sum p16 * v on the matrix cores for 128
+//           rows and one of pv_split key ranges.
+//   merge   the key ranges' partials added in order, and the gate.
 // Only the PV sum runs in another order than the reference (fp32 accumulation of exact products).
-
-#ifdef BKV_EXPERIMENT_TS
-#define PXTS(i) do { if (threadIdx.x == 0 && a.ts) a.ts[blockIdx.x * 16 + (i)] = (unsigned)wall_clock64(); } while (0)
-#else
-#define PXTS(i) do { } while (0)
-#endif
 
 // Workgroup barrier for LDS traffic only: every wave's LDS operations have completed, while its
 // global loads (prefetches a step or more ahead) stay in flight. __syncthreads() also releases
@@ -525,6 +523,307 @@ __device__ __forceinline__ void lds_barrier() {
 // memory-side cache, which non-temporal accesses bypass)
 __device__ __forceinline__ void st_sc4(float *p, float4 v) { *reinterpret_cast<float4 *>(p) = v; }
 __device__ __forceinline__ float4 ld_sc4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
+
+// the score kernels' work item: a run of NU units (NU x 4 queries) of one KV group and one of the
+// ksplit ranges of its key tiles (TILE keys each). Workgroups are dealt to the 8 XCDs round-robin;
+// when the grid is a multiple of 8 the index is permuted so that one XCD runs consecutive query
+// blocks of one (group, key range), which read the same K rows through that XCD's L2.
+// query block i of n in the order short, long, short, ... (a block's keys grow with its index): an
+// XCD's or a round's run of consecutive blocks then has about the same work whatever the start position
+__device__ __forceinline__ int px_mix(int i, int n) { return i & 1 ? n - 1 - (i >> 1) : i >> 1; }
+
+struct PxItem {
+  int u0, g, s, t0, t1;
+  uint32_t kend;                                   // keys 0 .. kend - 1 of the last unit's last query
+};
+template <int NU, int TILE>
+__device__ __forceinline__ PxItem px_item(const PrefillXArgs &a) {
+  const int n = gridDim.x, b = blockIdx.x;
+  const int wi = (n & 7) == 0 ? (b & 7) * (n >> 3) + (b >> 3) : b;
+  const int nub = (a.nqb + NU - 1) / NU;
+  PxItem p;
+  p.u0 = NU * px_mix(wi % nub, nub);
+  p.s = (wi / nub) % a.ksplit;
+  p.g = wi / (nub * a.ksplit);
+  p.kend = a.pos0 + (uint32_t)min(a.q_base + kPxQ * (p.u0 + NU), a.q_base + a.n_q);
+  const int nt = (int)((p.kend + TILE - 1) / TILE);
+  p.t0 = (int)((int64_t)p.s * nt / a.ksplit);
+  p.t1 = (int)((int64_t)(p.s + 1) * nt / a.ksplit);
+  return p;
+}
+
+// ---------------------------------------------------------------- q8_0 K scores on the matrix cores
+// The contract's inner sum (bkv_q8dot.h) is the fp32 rounding of the exact sum of q16 * int8 over a
+// block. fp16 MFMAs give it with two digits per q16, q = hi + lo: hi a multiple of u and lo a multiple
+// of t, where u is the smallest power of two with sum |hi| * 128 <= 2^24 u in every block of the row, and
+// sum |lo| * 128 <= 2^24 t. All products of a digit with bytes in [-128, 127] and all their partial sums
+// are then multiples of the digit's unit below 2^24 units: the MFMA's fp32 sums are exact in any
+// order, and fp32(hi sum + lo sum) is one fma with one rounding (lo is kept scaled by 2^8): one VALU
+// instruction per block and score, where int8 digits need two shifted adds, two conversions, an fma in
+// fp64 and its rounding. The row is scaled by a power of two so that u = 2^-2: hi <= 2^15, lo * 2^8 <= 2^5
+// in units above 2^-14, all fp16 normals; hi has at most 11 significant bits (a q16 of 2^10 u or more is
+// itself a multiple of u), lo at most 11 (it is q16 or a remainder of it).
+// A block whose lo is no multiple of such a t in some row (a q16 about 2^-16 of the row's largest or
+// less: one of a hundred rows of normal values has one) gets a third digit: lo a multiple of 2^-13 u,
+// lo2 = the rest, a multiple of 2^-26 u, kept scaled by 2^14. It costs a third MFMA, and its three sums
+// are combined in fp64 (below 2^53 units: exact) and rounded once. Rows that need more, or hold Inf / NaN,
+// take the fp64 VALU path.
+constexpr int kDigUnit = 2 * 8 * 64;               // 16-byte operands per unit: [pair j][block][lane]
+
+// Cooperative (256 threads, tid their index): the A operands of a unit's q rows (rows(i): the 4 head
+// rows of query i) in dig [pair][block][lane] (pair j: rows 4 i + 2 (h % 2) + digit for heads h = 2 j,
+// 2 j + 1 of query i) and lo2 [block][lane] (rows 4 i + h); lane l of an operand holds row l % 16, dims
+// 8 (l/16) .. + 7 of the block. ex[row 4 i + h]: the score's power of two. *flags: bit b set when block b
+// of any row has a third digit; *wide when the rows need the fp64 path. Both zeroed by the caller.
+template <typename ROWS>
+__device__ __forceinline__ void px_digits(int tid, const ROWS &rows, int qs, uint4 *dig, uint4 *lo2, float *ex,
+                                          unsigned *flags, unsigned *wide) {
+  const int r = tid >> 4, p = tid & 15, qi = r >> 2, h = r & 3;
+  const float *src = rows(qi) + (size_t)h * qs + 16 * p;
+  float x[16], s = 0.0f;
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 t = *reinterpret_cast<const float4 *>(src + 4 * i);
+    x[4 * i] = round_f16(t.x); x[4 * i + 1] = round_f16(t.y);
+    x[4 * i + 2] = round_f16(t.z); x[4 * i + 3] = round_f16(t.w);
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    bad = bad || !(fabsf(x[i]) <= 65504.0f);
+    s += fabsf(x[i]);
+  }
+  s += dpp<0xB1>(s);                               // the block's (two lanes hold one)
+  s = row16_max(s);                                // the row's largest
+  // S = s below 2^(E+1) (below 0.999 of it, for s's rounding and the u/2 that rounding adds to each hi):
+  // u = 2^(E-16); scaled so that u = 2^-2
+  const uint32_t sb = __float_as_uint(s);
+  const int E = s > 0.0f ? (int)(sb >> 23) - 127 + ((sb & 0x7FFFFFu) > 0x7FBFFFu ? 1 : 0) : 14;
+  bad = bad || E > 100;                            // (Inf / NaN rows: any finite scale)
+  const float up = bad ? 1.0f : __uint_as_float((uint32_t)(127 + 14 - E) << 23);
+  float lr[16], L = 0.0f;
+  h8 d0[2], d1[2], d2[2];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const float y = x[i] * up;                     // exact
+    const float hi = __builtin_rintf(y * 4.0f) * 0.25f;
+    lr[i] = y - hi;                                // exact, at most 2^-3
+    L += fabsf(lr[i]);
+    d0[i >> 3][i & 7] = (_Float16)hi;
+  }
+  L += dpp<0xB1>(L);
+  // t = 2^(exponent of L + 1 - 17), at least 2^-22: L * 128 < 2^24 t (L's fp32 rounding is far below the
+  // factor of up to 2 that the exponent leaves, except where L is within 2^-18 of a power of two: + 1)
+  const uint32_t lb = __float_as_uint(L) + 64u;
+  const float ti = __uint_as_float((uint32_t)(254 - max((int)(lb >> 23) + 1 - 17, 127 - 22)) << 23);   // 1 / t
+  bool fine = true;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) fine = fine && __builtin_rintf(lr[i] * ti) == lr[i] * ti;
+  const bool third = !(fine && dpp<0xB1>(fine ? 1.0f : 0.0f) == 1.0f);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const float lo = third ? __builtin_rintf(lr[i] * 32768.0f) * 0x1p-15f : lr[i];
+    const float l2 = (lr[i] - lo) * 16384.0f;      // exact, at most 2^-2
+    bad = bad || __builtin_rintf(l2 * 16384.0f) != l2 * 16384.0f;
+    d1[i >> 3][i & 7] = (_Float16)(lo * 256.0f);
+    d2[i >> 3][i & 7] = (_Float16)l2;
+  }
+  const int b = p >> 1;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int lq = 2 * (p & 1) + k, l = 16 * lq + 4 * qi + 2 * (h & 1);
+    uint4 *o = dig + ((h >> 1) * 8 + b) * 64;
+    o[l] = __builtin_bit_cast(uint4, d0[k]);
+    o[l + 1] = __builtin_bit_cast(uint4, d1[k]);
+    lo2[b * 64 + 16 * lq + r] = __builtin_bit_cast(uint4, d2[k]);
+  }
+  if (p == 0) ex[r] = 1.0f / up;
+  if (third) atomicOr(flags, 1u << b);
+  if (bad) atomicOr(wide, 1u);
+}
+
+// A workgroup scores UQ units against its range of key tiles (TILE keys each; UQ = 1: 128, else 64).
+// The tile's bytes become fp16 B operands in LDS once for all its units (2.5 instructions per 4 bytes:
+// at one unit per conversion they were a third of the kernel's VALU work), a tile ahead of the MFMAs:
+// lane (key, block) of the 8 waves loads 32 bytes and their scale while the tile before is scored, and
+// writes [key group][block][lane] operands (lanes XOR 8 (block % 2), so that the 8-key runs of two
+// blocks fall on different banks) and fp32 scales. Wave w scores unit w % UQ against NKG key groups.
+template <int UQ, bool PG>
+__global__ __launch_bounds__(512, 1) void prefill_score_q8_kernel(PrefillXArgs a) {
+  constexpr int TILE = UQ == 1 ? 2 * kPxTile : kPxTile, KGS = TILE / 16, NKG = KGS * UQ / 8, NC = TILE / 64;
+  const PxItem p = px_item<UQ, TILE>(a);
+  const int tid = threadIdx.x, lane = tid & 63, ql = lane >> 4, n16 = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), u = w % UQ, kg0 = NKG * (w / UQ);
+  __shared__ uint4 s_op[2][KGS * 8 * 64];          // first the units' digits (kDigUnit each), then the tiles
+  __shared__ __attribute__((aligned(16))) float s_sc[2][TILE][8];
+  __shared__ uint4 s_lo2[UQ][8 * 64];
+  __shared__ float s_ex[UQ][kPxRows];
+  __shared__ float s_red[8][kPxRows];
+  __shared__ unsigned s_flags[UQ], s_wide;
+  static_assert(sizeof(s_op) >= UQ * kDigUnit * 16, "the units' digits in the operand buffers");
+  uint4 *const op = &s_op[0][0];
+  if (tid < UQ) s_flags[tid] = 0u;
+  if (tid == 0) s_wide = 0u;
+  __syncthreads();
+  // (a workgroup's units past the slice's last one repeat that one: the same values stored twice)
+  auto unit = [&](int i) { return min(p.u0 + i, a.nqb - 1); };
+  const int qlast = a.q_base + a.n_q - 1;
+  auto qrows = [&](int q) {                        // the 4 q rows of chunk query q (clamped into the slice)
+    return a.q + ((size_t)min(q, qlast) * a.nh + p.g * kGqa) * a.qs;
+  };
+  for (int i = tid >> 8; i < UQ; i += 2) {
+    const int q0 = a.q_base + kPxQ * unit(i);
+    px_digits(tid & 255, [&](int q) { return qrows(q0 + q); }, a.qs, op + i * kDigUnit, s_lo2[i], s_ex[i], &s_flags[i],
+              &s_wide);
+  }
+  __syncthreads();
+  h8 da[2][8];                                     // the A operands of the wave's unit
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int b = 0; b < 8; ++b) da[j][b] = __builtin_bit_cast(h8, op[u * kDigUnit + (j * 8 + b) * 64 + lane]);
+  const int uq = kPxQ * unit(u) + ql;              // the lane's query in the slice
+  const int lim = uq < a.n_q ? (int)(a.pos0 + (uint32_t)(a.q_base + uq)) : -1;   // the last key it sees
+  const unsigned flags = (unsigned)__builtin_amdgcn_readfirstlane((int)s_flags[u]);
+  float mx[4], ex[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) { mx[k] = -INFINITY; ex[k] = s_ex[u][4 * ql + k]; }
+  constexpr int RB = row_bytes(BKV_Q8_0);
+  float *sc = a.sc + (((size_t)(p.g * a.nqb + unit(u)) * kPxQ + ql) * a.ld + n16) * kGqa;
+  // the scores of key group kg (keys key0 + 16 kg + lane % 16): lane l holds query l / 16's 4 heads;
+  // scaled, masked, into the scratch and the row maxima
+  auto emit = [&](uint32_t key0, int kg, const float (&r)[4]) {
+    const uint32_t j = key0 + (uint32_t)(16 * kg);
+    const bool live = (int)(j + n16) <= lim;
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] = live ? r[k] * a.scale : -INFINITY;
+      mx[k] = fmaxf(mx[k], v[k]);
+    }
+    st_sc4(sc + (size_t)j * kGqa, make_float4(v[0], v[1], v[2], v[3]));
+  };
+  if (s_wide == 0u) {
+    __syncthreads();                               // the digits are in registers
+    // this lane's (key, block) pairs of a tile: key 64 c + 8 w + lane % 8, block lane / 8
+    const int cn = lane & 7, cb = lane >> 3;
+    uint4 raw[NC][2];
+    uint32_t rsc[NC];
+    auto fetch = [&](int t) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const uint32_t key = min((uint32_t)(t * TILE + 64 * c + 8 * w + cn), p.kend - 1);
+        const int64_t ro = slot_t<PG>(a.L, key) * a.nkv + p.g;
+        const uint4 *src = reinterpret_cast<const uint4 *>(a.L.kd + ro * RB + 32 * cb);
+        raw[c][0] = src[0];
+        raw[c][1] = src[1];
+        rsc[c] = *reinterpret_cast<const uint16_t *>(a.L.ks + ro * kScaleRowBytes + 2 * cb);
+      }
+    };
+    auto convert = [&](int t) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int key = 64 * c + 8 * w + cn;       // of the tile
+        uint4 *o = op + (t & 1) * (KGS * 8 * 64) + ((key >> 4) * 8 + cb) * 64;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t w0 = (q & 1 ? raw[c][q >> 1].z : raw[c][q >> 1].x) ^ 0x80808080u;
+          const uint32_t w1 = (q & 1 ? raw[c][q >> 1].w : raw[c][q >> 1].y) ^ 0x80808080u;
+          o[(16 * q + (key & 15)) ^ (8 * (cb & 1))] =
+              make_uint4(as_u(bytes_h2<0x04010400u>(w0)), as_u(bytes_h2<0x04030402u>(w0)),
+                         as_u(bytes_h2<0x04010400u>(w1)), as_u(bytes_h2<0x04030402u>(w1)));
+        }
+        s_sc[t & 1][key][cb] = f16_to_f32(rsc[c]);
+      }
+    };
+    // every block's sums first (independent MFMAs), then the blocks with a third digit again, then the
+    // chains
+    auto score = [&](auto third, int t, int kg) {
+      const f4 z = {0.f, 0.f, 0.f, 0.f};
+      const uint4 *kop = op + (t & 1) * (KGS * 8 * 64) + kg * 8 * 64;
+      const float4 *sp = reinterpret_cast<const float4 *>(s_sc[t & 1][16 * kg + n16]);
+      const float4 sa = sp[0], sb = sp[1];
+      float x[8][4];
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const h8 kb = __builtin_bit_cast(h8, kop[b * 64 + (lane ^ (8 * (b & 1)))]);
+        const f4 s0 = mfma16(da[0][b], kb, z), s1 = mfma16(da[1][b], kb, z);
+        x[b][0] = __builtin_fmaf(s0[1], 0x1p-8f, s0[0]);
+        x[b][1] = __builtin_fmaf(s0[3], 0x1p-8f, s0[2]);
+        x[b][2] = __builtin_fmaf(s1[1], 0x1p-8f, s1[0]);
+        x[b][3] = __builtin_fmaf(s1[3], 0x1p-8f, s1[2]);
+      }
+      if constexpr (third.value) {
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+          if (flags & (1u << b)) {                 // (wave-uniform)
+            const h8 kb = __builtin_bit_cast(h8, kop[b * 64 + (lane ^ (8 * (b & 1)))]);
+            const f4 s0 = mfma16(da[0][b], kb, z), s1 = mfma16(da[1][b], kb, z);
+            const f4 s2 = mfma16(__builtin_bit_cast(h8, s_lo2[u][b * 64 + lane]), kb, z);
+            x[b][0] = (float)__builtin_fma((double)s2[0], 0x1p-14, __builtin_fma((double)s0[1], 0x1p-8, (double)s0[0]));
+            x[b][1] = (float)__builtin_fma((double)s2[1], 0x1p-14, __builtin_fma((double)s0[3], 0x1p-8, (double)s0[2]));
+            x[b][2] = (float)__builtin_fma((double)s2[2], 0x1p-14, __builtin_fma((double)s1[1], 0x1p-8, (double)s1[0]));
+            x[b][3] = (float)__builtin_fma((double)s2[3], 0x1p-14, __builtin_fma((double)s1[3], 0x1p-8, (double)s1[2]));
+          }
+        }
+      }
+      const float sf[8] = {sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, sb.z, sb.w};
+      float r[4];
+#pragma unroll
+      for (int b = 0; b < 8; ++b)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          r[k] = b == 0 ? __builtin_fmaf(sf[0], x[0][k], 0.0f) : __fadd_rn(r[k], __fmul_rn(sf[b], x[b][k]));
+#pragma unroll
+      for (int k = 0; k < 4; ++k) r[k] *= ex[k];
+      emit((uint32_t)(t * TILE), kg, r);
+    };
+    // tiles in descending key order (the sums kernel reads them ascending)
+    auto sweep = [&](auto third) {
+      fetch(p.t1 - 1);
+      convert(p.t1 - 1);
+      lds_barrier();
+      for (int t = p.t1 - 1; t >= p.t0; --t) {
+        if (t > p.t0) fetch(t - 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < NKG; ++c) score(third, t, kg0 + c);
+        __builtin_amdgcn_sched_barrier(0);
+        if (t > p.t0) convert(t - 1);              // (the buffer of tile t + 1, read before the last barrier)
+        lds_barrier();
+      }
+    };
+    if (p.t0 < p.t1) {                             // (the same barriers in both)
+      if (flags == 0u) sweep(std::false_type{});
+      else sweep(std::true_type{});
+    }
+  } else {
+    // the fp64 path: lane = key 16 kg + l%16 against query l/16's 4 heads
+    for (int t = p.t1 - 1; t >= p.t0; --t) {
+      for (int kg = kg0; kg < kg0 + NKG; ++kg) {
+        const uint32_t key = min((uint32_t)(t * TILE + 16 * kg + n16), p.kend - 1);
+        const int64_t ro = slot_t<PG>(a.L, key) * a.nkv + p.g;
+        float r[4];
+        q8_score_key_slow(reinterpret_cast<const uint32_t *>(a.L.kd + ro * RB),
+                          reinterpret_cast<const uint32_t *>(a.L.ks + ro * kScaleRowBytes), qrows(a.q_base + uq), a.qs, r);
+        emit((uint32_t)(t * TILE), kg, r);
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float m = row16_max(mx[k]);
+    if (n16 == 0) s_red[w][4 * ql + k] = m;
+  }
+  __syncthreads();
+  if (tid < UQ * kPxRows) {
+    const int i = tid / kPxRows, r = tid % kPxRows;
+    float m = s_red[i][r];
+#pragma unroll
+    for (int k = 1; k < 8 / UQ; ++k) m = fmaxf(m, s_red[i + UQ * k][r]);
+    a.mx[((size_t)(p.g * a.nqb + unit(i)) * a.ksplit + p.s) * kPxRows + r] = m;
+  }
+}
 
 // ---------------------------------------------------------------- fp16 K scores on the matrix cores
 // v_mfma_f32_16x16x1_4b_f32 computes, for 4 independent blocks b, D_b[i][j] += A_b[i] * B_b[j] with
@@ -542,276 +841,173 @@ __device__ __forceinline__ uint32_t word_of(const uint4 &v, int i) {
   return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
 }
 
-template <int KF, int VF, bool PG>
-__global__ __launch_bounds__(256, 2) void prefill_exact_kernel(PrefillXArgs a) {
+// A workgroup scores NU units against its range of 256-key tiles: one chain of 256 steps per (row,
+// key), acc = acc + q16*k in ascending dimension. Block b of the instruction is key group b (keys 16b ..
+// + 15 of the wave's 64), so one MFMA advances 64 keys x 16 rows; the wave's NU units are independent
+// chains on the same keys (each key's row, streamed 32 dimensions = 64 B at a time, one chunk ahead, goes
+// through the L1 once for all of them: with one unit and two key sets instead, the 64 lines a load
+// touches took as long as the MFMAs). s_qh[u][d4][i] = q16 of row i, dims 4 d4 .. + 3 (the lanes of one
+// row read the same float4).
+template <int NU, bool PG>
+__global__ __launch_bounds__(256, 2) void prefill_score_f16_kernel(PrefillXArgs a) {
+  const PxItem p = px_item<NU, kPxTile16>(a);
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), ql = lane >> 4;
+  __shared__ float4 s_qh[NU][(kHd / 4) * kPxRows];
+  __shared__ float s_red[4][NU][kPxRows];
+  // (a workgroup's units past the slice's last one repeat that one: the same values stored twice)
+  auto unit = [&](int i) { return min(p.u0 + i, a.nqb - 1); };
+  const int qlast = a.q_base + a.n_q - 1;
+#pragma unroll
+  for (int u = 0; u < NU; ++u)
+    for (int i = tid; i < (kHd / 4) * kPxRows; i += 256) {
+      const int r = i & 15, d4 = i >> 4;
+      const int qi = min(a.q_base + kPxQ * unit(u) + (r >> 2), qlast);
+      const float4 x = *reinterpret_cast<const float4 *>(a.q + ((size_t)qi * a.nh + p.g * kGqa + (r & 3)) * a.qs + 4 * d4);
+      s_qh[u][i] = make_float4(round_f16(x.x), round_f16(x.y), round_f16(x.z), round_f16(x.w));
+    }
+  __syncthreads();
+  float *sc[NU], mx[NU][4];
+  int lim[NU];                                     // the last key the lane's query sees
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int uq = kPxQ * unit(u) + ql;
+    lim[u] = uq < a.n_q ? (int)(a.pos0 + (uint32_t)(a.q_base + uq)) : -1;
+    sc[u] = a.sc + ((size_t)(p.g * a.nqb + unit(u)) * kPxQ + ql) * a.ld * kGqa;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) mx[u][k] = -INFINITY;
+  }
+  constexpr int RB = row_bytes(BKV_F16);
+  struct KChunk { uint4 d[4]; };               // [16 B]: dims 32c .. + 31 of the lane's key
+  auto load_chunk = [&](int T, int c, KChunk &k) {
+    const uint32_t key = min((uint32_t)(T * kPxTile16 + 64 * w + lane), p.kend - 1);
+    const uint4 *src = reinterpret_cast<const uint4 *>(a.L.kd + (slot_t<PG>(a.L, key) * a.nkv + p.g) * RB + 64 * c);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) k.d[q] = src[q];
+  };
+  auto chunk = [&](const KChunk &k, int c, fv16 (&d)[NU]) {
+#pragma unroll
+    for (int i4 = 0; i4 < 8; ++i4) {
+      float qa[NU][4];
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        const float4 q4 = s_qh[u][(8 * c + i4) * kPxRows + (lane & 15)];
+        qa[u][0] = q4.x; qa[u][1] = q4.y; qa[u][2] = q4.z; qa[u][3] = q4.w;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * i4 + e;      // dimension within the chunk: 16-bit half i of the 64 B
+        const uint32_t wv = word_of(k.d[i >> 3], (i >> 1) & 3);
+        const float kv = f16_to_f32((i & 1) ? (wv >> 16) : (wv & 0xFFFFu));
+#pragma unroll
+        for (int u = 0; u < NU; ++u) d[u] = mfma_k1(qa[u][e], kv, d[u]);
+      }
+    }
+  };
+  KChunk ka, kb;
+  // tiles in descending key order (the sums kernel reads them ascending); a wave without a key in the last
+  // one leaves it out (nothing reads past the last 64 keys)
+  int T = p.t1 - 1;
+  if (T >= p.t0 && (uint32_t)(T * kPxTile16 + 64 * w) >= p.kend) --T;
+  if (T >= p.t0) load_chunk(T, 0, ka);
+  for (; T >= p.t0; --T) {
+    fv16 d[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) d[u] = fv16{};
+#pragma unroll
+    for (int c = 0; c < kHd / 32; c += 2) {
+      load_chunk(T, c + 1, kb);
+      __builtin_amdgcn_sched_barrier(0);
+      chunk(ka, c, d);
+      __builtin_amdgcn_sched_barrier(0);
+      if (c + 2 < kHd / 32) load_chunk(T, c + 2, ka);
+      else load_chunk(max(T - 1, p.t0), 0, ka);
+      __builtin_amdgcn_sched_barrier(0);
+      chunk(kb, c + 1, d);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+#pragma unroll
+      for (int bq = 0; bq < 4; ++bq) {
+        const uint32_t j = (uint32_t)(T * kPxTile16 + 64 * w + 16 * bq + (lane & 15));
+        const bool live = (int)j <= lim[u];
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          v[k] = live ? d[u][4 * bq + k] * a.scale : -INFINITY;
+          mx[u][k] = v[k] > mx[u][k] ? v[k] : mx[u][k];
+        }
+        st_sc4(sc[u] + (size_t)j * kGqa, make_float4(v[0], v[1], v[2], v[3]));
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < NU; ++u)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float m = row16_max(mx[u][k]);
+      if ((lane & 15) == 0) s_red[w][u][4 * ql + k] = m;
+    }
+  __syncthreads();
+  if (tid < NU * kPxRows) {
+    const int i = tid / kPxRows, r = tid % kPxRows;
+    a.mx[((size_t)(p.g * a.nqb + unit(i)) * a.ksplit + p.s) * kPxRows + r] =
+        fmaxf(fmaxf(s_red[0][i][r], s_red[1][i][r]), fmaxf(s_red[2][i][r], s_red[3][i][r]));
+  }
+}
+
+// ---------------------------------------------------------------- exp and the serial sum
+// One unit per workgroup of NW waves. Waves 0..NW-2 form e for 64 (NW - 1) keys per step (one key per
+// thread, its 16 rows), store them over the scores and into an LDS tile [row][key]; the last wave adds
+// the previous step's e values of each row in key order (lane r: row r), four per LDS read and the next
+// reads in flight, so the serial chains run beside the exps. The chain bounds short chunks.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void prefill_sum_kernel(PrefillXArgs a) {
+  constexpr int NT = 64 * NW, kEK = 64 * (NW - 1);    // keys per step
+  constexpr int ES = kEK + 4;                         // floats per row of the tile (rows 4 banks apart)
   const int n = gridDim.x, b = blockIdx.x;
-  const int wi = (n & 7) == 0 ? (b & 7) * (n >> 3) + (b >> 3) : b;
-  const int qb = wi % a.nqb, g = wi / a.nqb;
-  const int q0 = a.q_base + qb * kPxQ;                   // first query (chunk index)
+  const int wp = (n & 7) == 0 ? (b & 7) * (n >> 3) + (b >> 3) : b;
+  const int qb = px_mix(wp % a.nqb, a.nqb);
+  const int wi = wp / a.nqb * a.nqb + qb;             // the unit
+  const int q0 = a.q_base + qb * kPxQ;                // first query (chunk index)
   const int nqv = min(kPxQ, a.q_base + a.n_q - q0);
-  const uint32_t kend = a.pos0 + (uint32_t)(q0 + nqv);  // keys 0 .. kend-1
-  const int ntile = (int)((kend + kPxTile - 1) / kPxTile);
+  const uint32_t kend = a.pos0 + (uint32_t)(q0 + nqv);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   float *sc = a.sc + (size_t)wi * a.ld * kPxRows;
-  // the causal limit of row r is pos0 + q0 + r/4 (rows of queries past the chunk see nothing)
-  const int lim0 = (int)(a.pos0 + (uint32_t)q0);
-
-  __shared__ float s_red[4][kPxRows];
-  __shared__ float s_m[kPxRows], s_sum[kPxRows];
-  __shared__ double s_t2[32];               // the exp table
-  constexpr int ES = kPxRows + 1;          // LDS row stride (floats) of the exp tile
-  constexpr int NT = kPxRows / 16;         // MFMA row tiles
-  constexpr int PR = kPxRows / 4;          // probabilities per thread per 64-key tile
-  constexpr int kBig2 = 2 * 256 * ES * 4, kBig3 = 2 * kPxRows * kPfRS + (VF ? 0 : 4 * 64 * kPfRS);
-  __shared__ __attribute__((aligned(16))) char s_big[kBig2 > kBig3 ? kBig2 : kBig3];
-
-  PXTS(0);
-#ifdef BKV_EXPERIMENT_TS
-  if (threadIdx.x == 0 && a.ts) a.ts[blockIdx.x * 16 + 8] = (unsigned)__smid();
-#endif
-  // ---------------------------------------------------------------- sweep 1: exact scores
-  // the rows' q16 in LDS: s_q[r][d], row r = query q0 + r/4 (clamped into the chunk), head 4g + r%4
+  __shared__ float s_m[kPxRows];
+  __shared__ double s_t2[32];                         // the exp table
+  __shared__ __attribute__((aligned(16))) float et[2][kPxRows * ES];
   if (tid < 32) s_t2[tid] = kExp2Tab[tid];
-  if constexpr (KF) {
-    // q8_0 K on the int8 matrix cores (bkv_q8dot.h): the digits of each of the workgroup's
-    // queries' 4 q rows in LDS, their A operands in registers. A wave scores its 64 keys of a tile
-    // as 4 key groups x 4 queries (one MFMA per block each) and transposes each key group's 4
-    // queries so that lane l holds rows 4(l/16) + k: query l/16, heads 0..3. Each key group's K
-    // bytes are requested a whole tile ahead (the rows come from HBM the first time any workgroup
-    // of the XCD reads them; the workgroups run nearly in step).
-    int8_t *s_lim = reinterpret_cast<int8_t *>(s_big);                    // [query][kLimBytes]
-    int *s_lt = reinterpret_cast<int *>(s_big + kPxQ * kLimBytes);        // [query][head]
-    static_assert(kPxQ * (kLimBytes + kGqa * 4) <= sizeof(s_big), "digits in the big LDS area");
-    __shared__ unsigned s_wide;
-    if (tid == 0) s_wide = 0u;
+  // the row maxima over the key ranges: 16 lanes of rows per NT / 16 ranges, through the exp tile
+  {
+    const float *mx = a.mx + (size_t)wi * a.ksplit * kPxRows + (tid & 15);
+    float m = -INFINITY;
+    for (int s = tid >> 4; s < a.ksplit; s += NT / 16) m = fmaxf(m, mx[s * kPxRows]);
+    et[0][tid] = m;
     __syncthreads();
-    const int qlast = a.q_base + a.n_q - 1;
-    auto qrows = [&](int jq) {                 // the 4 q rows of query jq (clamped into the chunk)
-      return a.q + ((size_t)min(q0 + jq, qlast) * a.nh + g * kGqa) * a.qs;
-    };
-#pragma unroll 1
-    for (int jq = 0; jq < kPxQ; ++jq)
-      q8lim_build(qrows(jq), a.qs, s_lim + jq * kLimBytes, s_lt + jq * kGqa, &s_wide, tid, 256);
-    __syncthreads();
-    const bool wide = s_wide != 0u;
-    long qa[kPxQ][8];
-    int qt[kPxQ];                              // the exponent of head l/16 of each query
-    {
-      Q8Lim t;
-#pragma unroll
-      for (int jq = 0; jq < kPxQ; ++jq) {
-        q8lim_load(s_lim + jq * kLimBytes, s_lt + jq * kGqa, t);
-#pragma unroll
-        for (int b = 0; b < 8; ++b) qa[jq][b] = t.a[b];
-        qt[jq] = t.t;
-      }
-    }
-    const int ql = lane >> 4, n16 = lane & 15;
-    const bool qlive = ql < nqv;
-    float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    constexpr int RB = row_bytes(BKV_Q8_0);
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    struct KG { long b[8]; u32x4 s; };        // one key group's B operands and the lane key's scales
-    // The loads are issued as inline asm, so that they stay where they are written (the compiler
-    // would sink them to the end of the tile) and its wait counting leaves them alone: kg_wait<N>
-    // waits until at most N vector memory operations issued after them are in flight, and names
-    // the registers, so no read of them moves above it.
-    auto load_kg = [&](uint32_t key0, int kg, KG &r) {
-      const uint32_t key = min(key0 + (uint32_t)(16 * kg + n16), kend - 1);
-      const int64_t ro = slot_t<PG>(a.L, key) * a.nkv + g;
-      const uint8_t *src = a.L.kd + ro * RB + 8 * ql;
-      const uint8_t *sp = a.L.ks + ro * kScaleRowBytes;
-#define BKV_LD2(i) asm volatile("global_load_dwordx2 %0, %1, off offset:" #i "*32" : "=v"(r.b[i]) : "v"(src) : "memory")
-      BKV_LD2(0); BKV_LD2(1); BKV_LD2(2); BKV_LD2(3); BKV_LD2(4); BKV_LD2(5); BKV_LD2(6); BKV_LD2(7);
-#undef BKV_LD2
-      asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(r.s) : "v"(sp) : "memory");
-    };
-    // the scores of key group kg of the tile at key0 (r[k]: row 4(l/16) + k), scaled and masked,
-    // into the scratch and the row maxima
-    auto emit = [&](uint32_t key0, int kg, const float (&r)[4]) {
-      const uint32_t j = key0 + (uint32_t)(16 * kg + n16);
-      const bool live = qlive && (int)j <= lim0 + ql;
-      float v[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        v[k] = live ? r[k] * a.scale : -INFINITY;
-        mx[k] = v[k] > mx[k] ? v[k] : mx[k];
-      }
-      st_sc4(sc + (size_t)j * kPxRows + 4 * ql, make_float4(v[0], v[1], v[2], v[3]));
-    };
-    if (!wide) {
-      // a whole tile ahead. When key group kg is used, what was issued after its loads is the store
-      // that followed them, the 3 later key groups' loads (9 each) and their stores: 31 operations
-      // (27 to 30 in the first tile, whose loads went out back to back), so 27 are left in flight.
-      KG kn[4];
-      auto kg_wait = [](KG &r) {
-        asm volatile("s_waitcnt vmcnt(27)"
-                     : "+v"(r.b[0]), "+v"(r.b[1]), "+v"(r.b[2]), "+v"(r.b[3]), "+v"(r.b[4]), "+v"(r.b[5]),
-                       "+v"(r.b[6]), "+v"(r.b[7]), "+v"(r.s)::"memory");
-      };
-#pragma unroll
-      for (int kg = 0; kg < 4; ++kg) load_kg((uint32_t)((ntile - 1) * kPxTile + 64 * w), kg, kn[kg]);
-      for (int t = ntile - 1; t >= 0; --t) {
-        const uint32_t key0 = (uint32_t)(t * kPxTile + 64 * w);
-#pragma unroll
-        for (int kg = 0; kg < 4; ++kg) {
-          KG &cur = kn[kg];
-          kg_wait(cur);
-          float r[4];
-          const uint4 scl = make_uint4(cur.s.x, cur.s.y, cur.s.z, cur.s.w);
-#pragma unroll
-          for (int jq = 0; jq < kPxQ; ++jq) r[jq] = q8_score16r(cur.b, scl, qa[jq], qt[jq]);
-          load_kg((uint32_t)(max(t - 1, 0) * kPxTile + 64 * w), kg, cur);
-          transpose_rows4(r);
-          emit(key0, kg, r);
-        }
-      }
-      // every load has landed before its registers are free again
-#pragma unroll
-      for (int kg = 0; kg < 4; ++kg)
-        asm volatile("s_waitcnt vmcnt(0)"
-                     : "+v"(kn[kg].b[0]), "+v"(kn[kg].b[1]), "+v"(kn[kg].b[2]), "+v"(kn[kg].b[3]), "+v"(kn[kg].b[4]),
-                       "+v"(kn[kg].b[5]), "+v"(kn[kg].b[6]), "+v"(kn[kg].b[7]), "+v"(kn[kg].s)::"memory");
-    } else {
-      // the wide path: lane = key 16 kg + l%16 against query l/16's 4 heads, fp64 inner sums
-      for (int t = ntile - 1; t >= 0; --t) {
-        const uint32_t key0 = (uint32_t)(t * kPxTile + 64 * w);
-        for (int kg = 0; kg < 4; ++kg) {
-          const uint32_t key = min(key0 + (uint32_t)(16 * kg + n16), kend - 1);
-          const int64_t ro = slot_t<PG>(a.L, key) * a.nkv + g;
-          float r[4];
-          q8_score_key_slow(reinterpret_cast<const uint32_t *>(a.L.kd + ro * RB),
-                            reinterpret_cast<const uint32_t *>(a.L.ks + ro * kScaleRowBytes), qrows(ql), a.qs, r);
-          emit(key0, kg, r);
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float m = row16_max(mx[k]);
-      if ((lane & 15) == 0) s_red[w][4 * ql + k] = m;
-    }
-  } else {
-    // fp16 K on the matrix cores: one chain of 256 steps per (row, key), acc = acc + q16*k in
-    // ascending dimension (each product exact in fp32, each step one fma). Block b of the
-    // instruction is key group b (keys 16b .. + 15 of a 64-key set), so one MFMA advances 64 keys x
-    // 16 rows; a wave runs two sets (keys 64w .. of the two halves of a 512-key super tile) as two
-    // independent chains, streaming each key's row 32 dimensions (64 B) at a time, one chunk ahead.
-    // s_qh[d4][i] = q16 of row i, dims 4 d4 .. + 3 (the lanes of one row read the same float4).
-    float4 *s_qh = reinterpret_cast<float4 *>(s_big);
-    {
-      const int qlast = a.q_base + a.n_q - 1;
-      for (int i = tid; i < (kHd / 4) * kPxRows; i += 256) {
-        const int r = i & 15, d4 = i >> 4;
-        const int qi = min(q0 + (r >> 2), qlast);
-        const float4 x = *reinterpret_cast<const float4 *>(a.q + ((size_t)qi * a.nh + g * kGqa + (r & 3)) * a.qs + 4 * d4);
-        s_qh[i] = make_float4(round_f16(x.x), round_f16(x.y), round_f16(x.z), round_f16(x.w));
-      }
+    if (tid < kPxRows) {
+      for (int i = 1; i < NT / 16; ++i) m = fmaxf(m, et[0][16 * i + tid]);
+      s_m[tid] = (tid >> 2) < nqv ? m : 0.f;
     }
     __syncthreads();
-    const int ql = lane >> 4;
-    const bool qlive = ql < nqv;
-    float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    const int nsup = (int)((kend + 2 * kPxTile - 1) / (2 * kPxTile));
-    constexpr int RB = row_bytes(BKV_F16);
-    struct KChunk { uint4 d[2][4]; };          // [set][16 B]: dims 32c .. + 31 of the lane's key
-    auto load_chunk = [&](int T, int c, KChunk &k) {
-#pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        const uint32_t key = min((uint32_t)(T * 2 * kPxTile + st * kPxTile + 64 * w + lane), kend - 1);
-        const uint4 *src = reinterpret_cast<const uint4 *>(a.L.kd + (slot_t<PG>(a.L, key) * a.nkv + g) * RB + 64 * c);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) k.d[st][q] = src[q];
-      }
-    };
-    auto chunk = [&](const KChunk &k, int c, fv16 (&d)[2]) {
-#pragma unroll
-      for (int i4 = 0; i4 < 8; ++i4) {
-        const float4 q4 = s_qh[(8 * c + i4) * kPxRows + (lane & 15)];
-        const float qa[4] = {q4.x, q4.y, q4.z, q4.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int i = 4 * i4 + e;      // dimension within the chunk: 16-bit half i of the 64 B
-#pragma unroll
-          for (int st = 0; st < 2; ++st) {
-            const uint32_t wv = word_of(k.d[st][i >> 3], (i >> 1) & 3);
-            d[st] = mfma_k1(qa[e], f16_to_f32((i & 1) ? (wv >> 16) : (wv & 0xFFFFu)), d[st]);
-          }
-        }
-      }
-    };
-    KChunk ka, kb;
-    load_chunk(nsup - 1, 0, ka);
-    // super tiles in descending key order (sweep 2 reads them ascending)
-    for (int T = nsup - 1; T >= 0; --T) {
-      fv16 d[2] = {fv16{}, fv16{}};
-#pragma unroll
-      for (int c = 0; c < kHd / 32; c += 2) {
-        load_chunk(T, c + 1, kb);
-        __builtin_amdgcn_sched_barrier(0);
-        chunk(ka, c, d);
-        __builtin_amdgcn_sched_barrier(0);
-        if (c + 2 < kHd / 32) load_chunk(T, c + 2, ka);
-        else load_chunk(max(T - 1, 0), 0, ka);
-        __builtin_amdgcn_sched_barrier(0);
-        chunk(kb, c + 1, d);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int st = 0; st < 2; ++st) {
-#pragma unroll
-        for (int bq = 0; bq < 4; ++bq) {
-          const uint32_t j = (uint32_t)(T * 2 * kPxTile + st * kPxTile + 64 * w + 16 * bq + (lane & 15));
-          const bool live = qlive && (int)j <= lim0 + ql;
-          float v[4];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            v[k] = live ? d[st][4 * bq + k] * a.scale : -INFINITY;
-            mx[k] = v[k] > mx[k] ? v[k] : mx[k];
-          }
-          st_sc4(sc + (size_t)j * kPxRows + 4 * ql, make_float4(v[0], v[1], v[2], v[3]));
-        }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float m = row16_max(mx[k]);
-      if ((lane & 15) == 0) s_red[w][4 * ql + k] = m;
-    }
   }
-  __syncthreads();
-  if (tid < kPxRows) {
-    float m = fmaxf(fmaxf(s_red[0][tid], s_red[1][tid]), fmaxf(s_red[2][tid], s_red[3][tid]));
-    s_m[tid] = (tid >> 2) < nqv ? m : 0.f;
-  }
-  __syncthreads();
-
-  PXTS(1);
-  // ---------------------------------------------------------------- sweep 2: exp and serial sum
-  // Waves 0..2 form e for 192 keys per step (one key per thread, its 16 rows) into an LDS tile
-  // while wave 3 adds the previous step's e values of each row in key order (lane r: row r), so
-  // the serial chains run beside the exps, and writes that tile over the scores (wave 3 reads no
-  // global memory, so its stores never hold up a wait for the exp waves' score loads).
-  constexpr int kEK = 192;                        // keys per step
-  float *et = reinterpret_cast<float *>(s_big);   // [2][kEK][ES]
   const int nstep = (int)((kend + kEK - 1) / kEK + 1) & ~1;   // even: the exp waves run steps in pairs
-  const uint32_t kscr = (uint32_t)(ntile * kPxTile);   // this workgroup's scratch keys
-  float sum = 0.f;
-  if (w < 3) {
+  const uint32_t kscr = (kend + kPxTile - 1) / kPxTile * kPxTile;   // scored keys
+  if (w < NW - 1) {
     float mrow[kPxRows];
 #pragma unroll
     for (int r = 0; r < kPxRows; ++r) mrow[r] = s_m[r];
     auto fetch = [&](int t, float4 (&v)[kPxRows / 4]) {
       const uint32_t j = min((uint32_t)(t * kEK + tid), kscr - 1);
-      const float *src = sc + (size_t)j * kPxRows;
+      const float *src = sc + (size_t)j * kGqa;
 #pragma unroll
-      for (int r4 = 0; r4 < kPxRows / 4; ++r4) v[r4] = ld_sc4(src + 4 * r4);
+      for (int q = 0; q < kPxQ; ++q) v[q] = ld_sc4(src + (size_t)q * a.ld * kGqa);
     };
     auto step = [&](int t, const float4 (&vc)[kPxRows / 4]) {
       const uint32_t j = (uint32_t)(t * kEK + tid);
-      float *eb = et + (t & 1) * kEK * ES + tid * ES;
+      float *eb = et[t & 1] + tid;
       const bool in = j < kscr;                    // keys past the scores: e = 0 (none are live)
-      // all 16 exps first, then the LDS stores: independent exps interleave (their table reads in
+      // all 16 exps first, then the stores: independent exps interleave (their table reads in
       // flight together) instead of each waiting out an LDS round trip behind the stores before it
       float ev[kPxRows], xv[kPxRows];
       bool slow[kPxRows], any = false;
@@ -833,185 +1029,117 @@ __global__ __launch_bounds__(256, 2) void prefill_exact_kernel(PrefillXArgs a) {
           if (slow[r]) ev[r] = exp_t_slow(xv[r]);
       }
 #pragma unroll
-      for (int r = 0; r < kPxRows; ++r) eb[r] = in ? ev[r] : 0.f;
+      for (int r = 0; r < kPxRows; ++r) eb[r * ES] = in ? ev[r] : 0.f;
       lds_barrier();
+      if (in) {
+        float *dst = sc + (size_t)j * kGqa;
+#pragma unroll
+        for (int q = 0; q < kPxQ; ++q)
+          st_sc4(dst + (size_t)q * a.ld * kGqa, make_float4(ev[4 * q], ev[4 * q + 1], ev[4 * q + 2], ev[4 * q + 3]));
+      }
     };
     // two register sets: each step's scores are requested two steps ahead
     float4 va[kPxRows / 4], vb[kPxRows / 4];
     fetch(0, va);
+    __builtin_amdgcn_sched_barrier(0);
     fetch(min(1, nstep - 1), vb);
     for (int t = 0; t < nstep; t += 2) {
       step(t, va);
+      __builtin_amdgcn_sched_barrier(0);
       fetch(min(t + 2, nstep - 1), va);
+      __builtin_amdgcn_sched_barrier(0);
       step(t + 1, vb);
+      __builtin_amdgcn_sched_barrier(0);
       fetch(min(t + 3, nstep - 1), vb);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
+    lds_barrier();
   } else {
     const int r = lane & 15;
-    for (int t = 0; t <= nstep; ++t) {
-      if (t > 0) {
-        const float *tile = et + ((t - 1) & 1) * kEK * ES;
-        if (lane < kPxRows) {
-          const float *col = tile + r;
-#pragma unroll 16
-          for (int k = 0; k < kEK; ++k) sum = sum + col[k * ES];
-        }
-        // the tile over the scores: key k's 16 rows as 4 float4, within the region's ld keys
-        float *dst = sc + (size_t)(t - 1) * kEK * kPxRows;
-        const int kmax = (int)min((int64_t)kEK, a.ld - (int64_t)(t - 1) * kEK);
+    float sum = 0.f;
+    lds_barrier();
+    for (int t = 0; t < nstep; ++t) {
+      const float4 *row = reinterpret_cast<const float4 *>(et[t & 1] + r * ES);
+      constexpr int B = 8;                            // reads in flight (32 keys)
+      float4 cur[B], nxt[B];
 #pragma unroll
-        for (int i = 0; i < kEK * kPxRows / 4 / 64; ++i) {
-          const int f = lane + 64 * i, k = f >> 2, r4 = f & 3;
-          const float *e4 = tile + k * ES + 4 * r4;
-          if (k < kmax) st_sc4(dst + 4 * f, make_float4(e4[0], e4[1], e4[2], e4[3]));
+      for (int i = 0; i < B; ++i) cur[i] = row[i];
+#pragma unroll
+      for (int k = 0; k < kEK / 4; k += B) {
+        if (k + B < kEK / 4)
+#pragma unroll
+          for (int i = 0; i < B; ++i) nxt[i] = row[k + B + i];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+          sum = sum + cur[i].x;
+          sum = sum + cur[i].y;
+          sum = sum + cur[i].z;
+          sum = sum + cur[i].w;
         }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < B; ++i) cur[i] = nxt[i];
       }
       lds_barrier();
     }
-    if (lane < kPxRows) s_sum[r] = (r >> 2) < nqv ? sum : 1.0f;
-  }
-  __syncthreads();
-
-  PXTS(2);
-  // ---------------------------------------------------------------- sweep 3: p16 and PV
-  if constexpr (VF) {
-    // q8_0 V: the exact sums go out, and prefill_pv64_kernel forms p16 and the PV for 64 rows at a
-    // time (each V byte converted once per 64 rows instead of per 16)
-    if (tid < kPxRows) a.sums[(size_t)wi * kPxRows + tid] = s_sum[tid];
-    return;
-  } else {
-  const int lr = lane & 15, lq = lane >> 4, kp = lane & 31, vh = lane >> 5;
-  char *s_p = s_big;                                              // [2][kPxRows][kPfRS]
-  char *vt_hi = s_big + 2 * kPxRows * kPfRS + w * (VF ? 2 : 1) * 64 * kPfRS;
-  char *vt_lo = vt_hi + (VF ? 64 * kPfRS : 0);
-  f4 o[4][NT];
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) o[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
-  const int nt64 = (int)((kend + kPfTile - 1) / kPfTile);
-  const int pk = tid >> 2, pr0 = PR * (tid & 3);   // this thread's probabilities: key pk, rows pr0..+PR
-  float ssum[PR], srcp[PR];
-#pragma unroll
-  for (int i = 0; i < PR; ++i) {
-    ssum[i] = s_sum[pr0 + i];
-    srcp[i] = 1.0f / ssum[i];
-  }
-  float4 en[PR / 4];
-  VRaw<VF> vrn;
-  auto load_tile = [&](int t) {
-    const float *src = sc + ((size_t)t * kPfTile + pk) * kPxRows + pr0;
-#pragma unroll
-    for (int i = 0; i < PR / 4; ++i) en[i] = ld_sc4(src + 4 * i);
-    const uint32_t ka = min((uint32_t)(t * kPfTile + 2 * kp), kend - 1);
-    const uint32_t kb = min((uint32_t)(t * kPfTile + 2 * kp + 1), kend - 1);
-    load_v<VF, PG>(a.L, a.nkv, g, ka, kb, w, vh, vrn);
-  };
-  // tiles in descending key order (the PV sum's order is free): the last-written exp values first
-  load_tile(nt64 - 1);
-  for (int t = nt64 - 1; t >= 0; --t) {
-    char *pb = s_p + (t & 1) * kPxRows * kPfRS;
-    float ev[PR];
-#pragma unroll
-    for (int i = 0; i < PR / 4; ++i) {
-      ev[4 * i] = en[i].x; ev[4 * i + 1] = en[i].y; ev[4 * i + 2] = en[i].z; ev[4 * i + 3] = en[i].w;
-    }
-    const VRaw<VF> vr = vrn;
-    load_tile(max(t - 1, 0));   // in flight during this tile
-#pragma unroll
-    for (int i = 0; i < PR; ++i) {
-      const _Float16 h = (_Float16)div_by_sum(ev[i], ssum[i], srcp[i]);
-      *reinterpret_cast<_Float16 *>(pb + (pr0 + i) * kPfRS + 2 * pk) = h;
-    }
-    put_vt<VF>(vr, kp, vh, vt_hi, vt_lo);
-    __syncthreads();
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      h8 bp[NT];
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-        bp[nt] = *reinterpret_cast<const h8 *>(pb + (16 * nt + lr) * kPfRS + 2 * (32 * ks + 8 * lq));
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) {
-        const h8 ah = *reinterpret_cast<const h8 *>(vt_hi + (16 * mt + lr) * kPfRS + 2 * (32 * ks + 8 * lq));
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) o[mt][nt] = mfma16(ah, bp[nt], o[mt][nt]);
-        if constexpr (VF) {
-          const h8 al = *reinterpret_cast<const h8 *>(vt_lo + (16 * mt + lr) * kPfRS + 2 * (32 * ks + 8 * lq));
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt) o[mt][nt] = mfma16(al, bp[nt], o[mt][nt]);
-        }
-      }
-    }
-  }
-  PXTS(3);
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int r = 16 * nt + lr;
-    if ((r >> 2) >= nqv) continue;
-    const size_t row = (size_t)(q0 + (r >> 2)) * a.nh + g * kGqa + (r & 3);
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      const int d = 64 * w + 16 * mt + 4 * lq;
-      const float4 v = make_float4(o[mt][nt][0], o[mt][nt][1], o[mt][nt][2], o[mt][nt][3]);
-      *reinterpret_cast<float4 *>(a.out + row * kHd + d) = v;
-      if (a.gate) {
-        const float4 gt = *reinterpret_cast<const float4 *>(a.gate + row * a.gs + d);
-        float4 og;
-        og.x = v.x * (1.0f / (1.0f + exp_cr(-gt.x)));
-        og.y = v.y * (1.0f / (1.0f + exp_cr(-gt.y)));
-        og.z = v.z * (1.0f / (1.0f + exp_cr(-gt.z)));
-        og.w = v.w * (1.0f / (1.0f + exp_cr(-gt.w)));
-        *reinterpret_cast<float4 *>(a.out_gated + row * kHd + d) = og;
-      }
-    }
-  }
+    if (lane < kPxRows) a.sums[(size_t)wi * kPxRows + r] = (r >> 2) < nqv ? sum : 1.0f;
   }
 }
 
-// ---------------------------------------------------------------- the exact prefill's PV, q8_0 V
-// 16 queries (64 rows: query i, head h at row 4 i + h) of one KV group over one half of their key
-// tiles: p16 = f16(e / sum) from the exact kernel's e scratch and sums (the reference's P16,
+// out_gated = v * 1/(1 + exp(-gate)) for dims d .. + 3 of the chunk's row
+__device__ __forceinline__ void px_gate(const PrefillXArgs &a, size_t row, int d, const float4 &v) {
+  const float4 gt = *reinterpret_cast<const float4 *>(a.gate + row * a.gs + d);
+  float4 og;
+  og.x = v.x * (1.0f / (1.0f + exp_cr(-gt.x)));
+  og.y = v.y * (1.0f / (1.0f + exp_cr(-gt.y)));
+  og.z = v.z * (1.0f / (1.0f + exp_cr(-gt.z)));
+  og.w = v.w * (1.0f / (1.0f + exp_cr(-gt.w)));
+  *reinterpret_cast<float4 *>(a.out_gated + row * kHd + d) = og;
+}
+
+// ---------------------------------------------------------------- PV
+// kPvQ queries (128 rows: query i, head h at row 4 i + h) of one KV group over one of pv_split ranges
+// of their key tiles: p16 = f16(e / sum) from the sums kernel's e and sums (the reference's P16,
 // attn_vk.h:190-200), out^T = V^T . P^T on v_mfma_f32_16x16x32_f16, wave w of 8 owning dims
-// 32 w .. + 31 (one q8_0 block). Each 64-key tile of V goes into LDS by direct-to-LDS loads (one
-// 1 KiB block of 4 keys per load, two per wave) in the blocked layout of bkv_pv8.h; lane l then reads
-// A row i = l%16 of dimension tile mt (dim 32 w + 16 mt + i) over keys 8(l/16) .. + 7 of each 32-key
-// half with one ds_read_b64_tr_b8, and the exact fp16 split of d*b (hi = f16(d*b), lo = d*b - hi)
-// forms the operands, shared by the 64 rows. The two halves' partials are added in a fixed order by
-// prefill_pv_merge_kernel.
-template <bool PG>
+// 32 w .. + 31 (one q8_0 block). Each 64-key tile of V goes into LDS by direct-to-LDS loads, 1 KiB
+// blocks of 4 keys x 256 bytes (q8_0: whole rows; fp16: the rows' first, then their second halves) in
+// the blocked layout of bkv_pv8.h; a lane then reads its A operand (8 keys of one dim) with transposed
+// LDS reads. q8_0: one ds_read_b64_tr_b8, and the exact fp16 split of d*b (hi = f16(d*b), lo = d*b -
+// hi) forms two operands shared by the 128 rows. fp16: two ds_read_b64_tr_b16. The ranges' partials are
+// added in a fixed order by prefill_pv_merge_kernel.
+template <int VF, bool PG>
 __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
-  constexpr int R = kGqa * kPvQ;                   // rows, kPvQ / kPxQ exact-kernel workgroups' worth
+  constexpr int R = kGqa * kPvQ;                   // rows, kPvQ / kPxQ units' worth
   constexpr int NTR = R / 16;                      // MFMA row tiles
   constexpr int RPW = R / 8;                       // rows per wave of the P tile
-  static_assert(RPW % 4 == 0 && kPxRows % RPW == 0 || RPW % kPxRows == 0, "a wave's rows in whole float4s");
+  static_assert(RPW == kPxRows, "a wave's rows are one unit");
   const int n = gridDim.x, b = blockIdx.x;
   const int nqp = (a.n_q + kPvQ - 1) / kPvQ;
   const int wb = (n & 7) == 0 ? (b & 7) * (n >> 3) + (b >> 3) : b;
-  const int qb = wb % nqp, sp = (wb / nqp) % kPvSplit, g = wb / (kPvSplit * nqp);
+  const int qb = px_mix(wb % nqp, nqp), sp = (wb / nqp) % a.pv_split, g = wb / (a.pv_split * nqp);
   const int q0 = a.q_base + kPvQ * qb;             // chunk index of the first query
   const int nqv = min(kPvQ, a.q_base + a.n_q - q0);
   const uint32_t kend = a.pos0 + (uint32_t)(q0 + nqv);
   const int ntl = (int)((kend + kPfTile - 1) / kPfTile);
-  const int t0 = sp * ntl / kPvSplit, t1 = (sp + 1) * ntl / kPvSplit;
+  const int t0 = (int)((int64_t)sp * ntl / a.pv_split), t1 = (int)((int64_t)(sp + 1) * ntl / a.pv_split);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lq = lane >> 4;
-  __shared__ __attribute__((aligned(16))) char s_p[2][R * kPfRS];   // P tiles [row][64 keys] fp16
-  // this thread's probabilities: key pk of a tile, rows RPW w .. + RPW - 1 (of exact-kernel
-  // workgroup xq, whose scratch holds their e up to its own last key kx); the wave's sums in scalar
-  // registers
+  __shared__ __attribute__((aligned(16))) float s_pbuf[2 * R * kPfRS / 4];   // P tiles [row][64 keys] fp16
+  char *s_p = reinterpret_cast<char *>(s_pbuf);
+  // this thread's probabilities: key pk of a tile, the 16 rows of unit xr (whose scratch holds their e
+  // up to its own last key kx); the wave's sums in scalar registers
   const int pk = lane;
-  const int xr = (R / kPxRows) * qb + RPW * w / kPxRows, roff = RPW * w % kPxRows;
+  const int xr = kPvQ / kPxQ * qb + w;
   const int xq = min(xr, a.nqb - 1);
   const bool pv = kPxQ * xr < a.n_q;
   const uint32_t kx = a.pos0 + (uint32_t)min(a.q_base + kPxQ * xr + kPxQ, a.q_base + a.n_q);
   const size_t xw = (size_t)g * a.nqb + xq;
-  const float *esrc = a.sc + xw * a.ld * kPxRows + roff;
+  const float *esrc = a.sc + xw * a.ld * kPxRows;
   float ssum[RPW], srcp[RPW];
 #pragma unroll
   for (int i = 0; i < RPW; ++i) {
     ssum[i] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
-                                            __builtin_bit_cast(int, a.sums[xw * kPxRows + roff + i])));
+                                            __builtin_bit_cast(int, a.sums[xw * kPxRows + i])));
     srcp[i] = 1.0f / ssum[i];
   }
   f4 o[2][NTR];
@@ -1019,17 +1147,25 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
   for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
     for (int nt = 0; nt < NTR; ++nt) o[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
-  // V tiles: three LDS buffers (tile t in buffer t % 3), each 16 blocks of 4 keys (block i at 1024 i,
-  // 16-byte chunk c of its row r at 64 (c ^ (i & 3)) + 16 r: the rows one transposed read takes
-  // spread over the banks)
-  __shared__ __attribute__((aligned(1024))) char s_v[3][16384];
+  // V tiles: three LDS buffers (tile t in buffer t % 3), each of 16 (fp16: 32) blocks of 1 KiB: 16-byte
+  // chunk c of row r of block i at 64 (c ^ swizzle(i)) + 16 r, so that the rows one transposed read
+  // takes spread over the banks
+  constexpr int VB = VF ? 16384 : 32768;           // bytes per tile
+  __shared__ __attribute__((aligned(1024))) char s_v[3][VB];
   const uint32_t vbase = __builtin_amdgcn_readfirstlane(lds_addr(s_v));
-  // the lane's read address in a tile buffer for key half ks (dim tile: XOR 64 (2 w + mt))
+  // the lane's read address in a tile buffer for key half ks (q8_0: dim tile mt by XOR 64 (2 w + mt);
+  // fp16: dim tile mt by XOR 128 (2 (w % 4) + mt), the second 4 of its 8 keys one block on)
   uint32_t vrd[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
-    const int j = lr >> 1, bl = 8 * ks + 2 * lq + (j >> 2);
-    vrd[ks] = (uint32_t)(1024 * bl + 16 * (j & 3) + 8 * (lane & 1) + 64 * (bl & 3));
+    if constexpr (VF) {
+      const int j = lr >> 1, bl = 8 * ks + 2 * lq + (j >> 2);
+      vrd[ks] = (uint32_t)(1024 * bl + 16 * (j & 3) + 8 * (lane & 1) + 64 * (bl & 3));
+    } else {
+      const int bl = 8 * ks + 2 * lq;
+      vrd[ks] = (uint32_t)(1024 * (bl + 16 * (w >> 2)) + 64 * (((lane >> 1) & 1) ^ (2 * (lq & 3))) + 16 * (lr >> 2) +
+                           8 * (lane & 1));
+    }
   }
   // (the loaded values are kept raw until the tile uses them: any arithmetic on them here would
   // make the wave wait for the loads at once)
@@ -1042,30 +1178,36 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
   auto load_tile = [&](int tt, PvIn &in) {
     const int t = min(tt, t1 - 1);
     const uint32_t j = (uint32_t)(t * kPfTile + pk);
-    const float *src = esrc + (size_t)min(j, kx - 1) * kPxRows;
+    const float *src = esrc + (size_t)min(j, kx - 1) * kGqa;
 #pragma unroll
-    for (int i = 0; i < RPW / 4; ++i) in.en[i] = ld_sc4(src + 4 * i);
+    for (int i = 0; i < RPW / 4; ++i) in.en[i] = ld_sc4(src + (size_t)i * a.ld * kGqa);
     in.live = pv && j < kx && tt < t1;
-    // one scale load per lane: lane l%16 of each 16-lane row loads key (l%16 / 8, l%8)'s, and the row
-    // shares them by DPP broadcasts in the tile
-    const uint32_t skey = min((uint32_t)(t * kPfTile + 32 * (lr >> 3) + 8 * lq + (lr & 7)), kend - 1);
-    in.vs = *reinterpret_cast<const uint16_t *>(a.L.vs + (slot_t<PG>(a.L, skey) * a.nkv + g) * kScaleRowBytes + 2 * w);
+    if constexpr (VF) {
+      // one scale load per lane: lane l%16 of each 16-lane row loads key (l%16 / 8, l%8)'s, and the row
+      // shares them by DPP broadcasts in the tile
+      const uint32_t skey = min((uint32_t)(t * kPfTile + 32 * (lr >> 3) + 8 * lq + (lr & 7)), kend - 1);
+      in.vs = *reinterpret_cast<const uint16_t *>(a.L.vs + (slot_t<PG>(a.L, skey) * a.nkv + g) * kScaleRowBytes + 2 * w);
+    }
   };
-  // the V rows of tile tt (clamped as above) into buffer tt % 3: wave w loads blocks 2 w, 2 w + 1
-  // (keys 4 i + lane % 4, chunk (lane / 4) ^ (i % 4) at 16 lane)
+  // the V rows of tile tt (clamped as above) into buffer tt % 3: wave w loads the blocks i of keys
+  // 4 i .. + 3 for i = 2 w, 2 w + 1 (lane: key 4 i + lane % 4, chunk (lane / 4) ^ swizzle at 16 lane)
+  constexpr int ND = VF ? 2 : 4;                    // loads per wave
   auto dma_tile = [&](int tt) {
     const int t = min(tt, t1 - 1);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int i = 2 * w + u;
+    for (int u = 0; u < ND; ++u) {
+      const int i = 2 * w + (u & 1);                // block of keys; u / 2: half of an fp16 row
       const uint32_t key = min((uint32_t)(t * kPfTile + 4 * i + (lane & 3)), kend - 1);
-      const uint8_t *src = a.L.vd + (slot_t<PG>(a.L, key) * a.nkv + g) * kHd + 16 * ((lane >> 2) ^ (i & 3));
+      const int sw = VF ? (i & 3) : 2 * ((i >> 1) & 3);
+      const uint8_t *src = a.L.vd + (slot_t<PG>(a.L, key) * a.nkv + g) * row_bytes(VF ? BKV_Q8_0 : BKV_F16) +
+                           256 * (u >> 1) + 16 * ((lane >> 2) ^ sw);
       asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src),
-                   "s"(__builtin_amdgcn_readfirstlane(vbase + 16384u * (uint32_t)(tt % 3) + 1024u * i)) : "memory", "m0");
+                   "s"(__builtin_amdgcn_readfirstlane(vbase + (uint32_t)VB * (uint32_t)(tt % 3) + 1024u * (i + 16 * (u >> 1))))
+                   : "memory", "m0");
     }
   };
   auto tile = [&](int t, const PvIn &in) {
-    char *pb = s_p[t & 1];
+    char *pb = s_p + (t & 1) * (R * kPfRS);
     float ev[RPW];
 #pragma unroll
     for (int i = 0; i < RPW / 4; ++i) {
@@ -1078,40 +1220,50 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
     }
     // the block scales of the lane's 16 keys: key (ks, c) from lane 8 ks + c of its row
     uint32_t vsk[16];
+    if constexpr (VF) {
 #define BKV_BC(i) vsk[i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)in.vs, 0x150 + (i), 0xF, 0xF, false)
-    BKV_BC(0); BKV_BC(1); BKV_BC(2); BKV_BC(3); BKV_BC(4); BKV_BC(5); BKV_BC(6); BKV_BC(7);
-    BKV_BC(8); BKV_BC(9); BKV_BC(10); BKV_BC(11); BKV_BC(12); BKV_BC(13); BKV_BC(14); BKV_BC(15);
+      BKV_BC(0); BKV_BC(1); BKV_BC(2); BKV_BC(3); BKV_BC(4); BKV_BC(5); BKV_BC(6); BKV_BC(7);
+      BKV_BC(8); BKV_BC(9); BKV_BC(10); BKV_BC(11); BKV_BC(12); BKV_BC(13); BKV_BC(14); BKV_BC(15);
 #undef BKV_BC
+    }
     // this wave's V rows of tile t have landed when at most the loads issued after them are in
-    // flight: tile t + 1's register loads (NL) and rows (2), tile t + 2's register loads (NL)
-    constexpr int NL = RPW / 4 + 1;
-    static_assert(2 * NL + 2 == 8 || 2 * NL + 2 == 12, "the wait count below");
-    if constexpr (2 * NL + 2 == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    // flight: tile t + 1's register loads (NL) and rows (ND), tile t + 2's register loads (NL)
+    constexpr int NL = RPW / 4 + (VF ? 1 : 0);
+    static_assert(2 * NL + ND == 12, "the wait count below");
+    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
     lds_barrier();                                  // the P tile and every wave's V rows of tile t
     dma_tile(t + 2);                                // (its buffer's last readers, tile t - 1, are done)
-    const uint32_t vb = vbase + 16384u * (uint32_t)(t % 3);
+    const uint32_t vb = vbase + (uint32_t)VB * (uint32_t)(t % 3);
     // the A operands (registers only): pair p of key half ks holds keys 2p, 2p+1
     h8 ah[2][2], al[2][2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
-        const v2i_t bv = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-            (__attribute__((address_space(3))) v2i_t *)(uintptr_t)((vb + vrd[ks]) ^ (uint32_t)(64 * (2 * w + mt))));
-        constexpr uint32_t kSel[4] = {0x0C010C00u, 0x0C030C02u, 0x0C050C04u, 0x0C070C06u};
-        uint32_t hw[4], lw[4];
+        if constexpr (VF) {
+          const v2i_t bv = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+              (__attribute__((address_space(3))) v2i_t *)(uintptr_t)((vb + vrd[ks]) ^ (uint32_t)(64 * (2 * w + mt))));
+          constexpr uint32_t kSel[4] = {0x0C010C00u, 0x0C030C02u, 0x0C050C04u, 0x0C070C06u};
+          uint32_t hw[4], lw[4];
 #pragma unroll
-        for (int pp = 0; pp < 4; ++pp) {
-          const uint32_t bw = __builtin_amdgcn_perm((uint32_t)bv.y, (uint32_t)bv.x, kSel[pp]) ^ 0x64806480u;
-          const h2 x = as_h2(bw) - h2{(_Float16)1152.0f, (_Float16)1152.0f};
-          h2 hi, lo;
-          split_prod(x, as_h2(vsk[8 * ks + 2 * pp] | (vsk[8 * ks + 2 * pp + 1] << 16)), hi, lo);
-          hw[pp] = as_u(hi);
-          lw[pp] = as_u(lo);
+          for (int pp = 0; pp < 4; ++pp) {
+            const uint32_t bw = __builtin_amdgcn_perm((uint32_t)bv.y, (uint32_t)bv.x, kSel[pp]) ^ 0x64806480u;
+            const h2 x = as_h2(bw) - h2{(_Float16)1152.0f, (_Float16)1152.0f};
+            h2 hi, lo;
+            split_prod(x, as_h2(vsk[8 * ks + 2 * pp] | (vsk[8 * ks + 2 * pp + 1] << 16)), hi, lo);
+            hw[pp] = as_u(hi);
+            lw[pp] = as_u(lo);
+          }
+          ah[ks][mt] = __builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3]));
+          al[ks][mt] = __builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3]));
+        } else {
+          // keys 8 lq .. + 3 of the half from one block, + 4 .. + 7 from the next (the same swizzle)
+          const uint32_t ad = (vb + vrd[ks]) ^ (uint32_t)(128 * (2 * (w & 3) + mt));
+          const v4s_t r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)ad);
+          const v4s_t r1 =
+              __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)(ad + 1024u));
+          ah[ks][mt] = __builtin_bit_cast(h8, (v8s_t){r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]});
         }
-        ah[ks][mt] = __builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3]));
-        al[ks][mt] = __builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3]));
       }
     }
 #pragma unroll
@@ -1122,7 +1274,7 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
           o[mt][nt] = mfma16(ah[ks][mt], bp, o[mt][nt]);
-          o[mt][nt] = mfma16(al[ks][mt], bp, o[mt][nt]);
+          if constexpr (VF) o[mt][nt] = mfma16(al[ks][mt], bp, o[mt][nt]);
         }
       }
     }
@@ -1146,59 +1298,119 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last rows landed before the LDS is released
   }
-  // lane l holds out^T[dim 32 w + 16 mt + 4(l/16) + r][row 16 nt + l%16] in o[mt][nt][r]
-  float *part = a.part + (size_t)sp * kPxSlice * a.nh * kHd;
+  // lane l holds out^T[dim 32 w + 16 mt + 4(l/16) + r][row 16 nt + l%16] in o[mt][nt][r]: the range's
+  // partial, or (one range) the output
+  const bool whole = a.pv_split == 1;
+  float *part = whole ? a.out + (size_t)a.q_base * a.nh * kHd : a.part + (size_t)sp * a.n_q * a.nh * kHd;
 #pragma unroll
   for (int nt = 0; nt < NTR; ++nt) {
     const int r = 16 * nt + lr;
     if ((r >> 2) >= nqv) continue;
     const size_t row = (size_t)(q0 - a.q_base + (r >> 2)) * a.nh + g * kGqa + (r & 3);
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-      *reinterpret_cast<float4 *>(part + row * kHd + 32 * w + 16 * mt + 4 * lq) =
-          make_float4(o[mt][nt][0], o[mt][nt][1], o[mt][nt][2], o[mt][nt][3]);
+    for (int mt = 0; mt < 2; ++mt) {
+      const int d = 32 * w + 16 * mt + 4 * lq;
+      const float4 v = make_float4(o[mt][nt][0], o[mt][nt][1], o[mt][nt][2], o[mt][nt][3]);
+      *reinterpret_cast<float4 *>(part + row * kHd + d) = v;
+      if (whole && a.gate) px_gate(a, (size_t)a.q_base * a.nh + row, d, v);
+    }
   }
 }
 
-// out = partial of the first key half + partial of the second (in that order), and the gate
+// out = the key ranges' partials added in range order, and the gate
 __global__ __launch_bounds__(256) void prefill_pv_merge_kernel(PrefillXArgs a) {
   const size_t n4 = (size_t)a.n_q * a.nh * (kHd / 4);
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n4) return;
-  float4 v = reinterpret_cast<const float4 *>(a.part)[i];
-#pragma unroll
-  for (int s = 1; s < kPvSplit; ++s) {           // the key ranges in order
-    const float4 y = reinterpret_cast<const float4 *>(a.part + (size_t)s * kPxSlice * a.nh * kHd)[i];
+  const float4 *pp = reinterpret_cast<const float4 *>(a.part) + i;
+  float4 v = pp[0];
+#pragma unroll 8
+  for (int s = 1; s < a.pv_split; ++s) {
+    const float4 y = pp[(size_t)s * n4];
     v = make_float4(v.x + y.x, v.y + y.y, v.z + y.z, v.w + y.w);
   }
-  const size_t row = i / (kHd / 4), d = 4 * (i % (kHd / 4));
-  const size_t grow = (size_t)a.q_base * a.nh + row;             // row of the whole chunk
+  const size_t grow = (size_t)a.q_base * a.nh + i / (kHd / 4);   // row of the whole chunk
+  const int d = 4 * (int)(i % (kHd / 4));
   *reinterpret_cast<float4 *>(a.out + grow * kHd + d) = v;
-  if (a.gate) {
-    const float4 gt = *reinterpret_cast<const float4 *>(a.gate + grow * a.gs + d);
-    float4 og;
-    og.x = v.x * (1.0f / (1.0f + exp_cr(-gt.x)));
-    og.y = v.y * (1.0f / (1.0f + exp_cr(-gt.y)));
-    og.z = v.z * (1.0f / (1.0f + exp_cr(-gt.z)));
-    og.w = v.w * (1.0f / (1.0f + exp_cr(-gt.w)));
-    *reinterpret_cast<float4 *>(a.out_gated + grow * kHd + d) = og;
-  }
+  if (a.gate) px_gate(a, grow, d, v);
 }
 
-hipError_t launch_prefill_exact(const PrefillXArgs &a, int kf, int vf, hipStream_t st) {
-  const int grid = a.nkv * a.nqb;
-  const bool pg = a.L.page != 0;
-  BKV_FMT_SWITCH(kf, vf, {
-    if (pg) hipLaunchKernelGGL((prefill_exact_kernel<KF_, VF_, true>), dim3(grid), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((prefill_exact_kernel<KF_, VF_, false>), dim3(grid), dim3(256), 0, st, a);
-  });
-  if (vf == BKV_Q8_0) {
-    const int pgrid = a.nkv * kPvSplit * ((a.n_q + kPvQ - 1) / kPvQ);
-    if (pg) hipLaunchKernelGGL(prefill_pv64_kernel<true>, dim3(pgrid), dim3(512), 0, st, a);
-    else hipLaunchKernelGGL(prefill_pv64_kernel<false>, dim3(pgrid), dim3(512), 0, st, a);
-    const size_t n4 = (size_t)a.n_q * a.nh * (kHd / 4);
-    hipLaunchKernelGGL(prefill_pv_merge_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, a);
+// How many key ranges to split each of `items` work items of `tiles` key tiles into: the count whose
+// rounds of `slots` resident workgroups take least, a workgroup costing `fixed` (its prologue and
+// epilogue) plus `tile` per tile, and `merge` per range where there are several (ns).
+static int px_ranges(int64_t items, int64_t tiles, int64_t slots, int64_t tile, int64_t fixed, int64_t merge, int64_t most) {
+  int64_t best = 1, cost = INT64_MAX;
+  for (int64_t ks = 1; ks <= std::min<int64_t>({tiles, most, 128}); ++ks) {
+    const int64_t c = (items * ks + slots - 1) / slots * ((tiles + ks - 1) / ks * tile + fixed) + (ks > 1 ? ks * merge : 0);
+    if (c < cost) {
+      cost = c;
+      best = ks;
+    }
   }
+  return (int)best;
+}
+
+hipError_t launch_prefill_exact(PrefillXArgs a, int kf, int vf, hipStream_t st) {
+  const bool pg = a.L.page != 0;
+  const int64_t kmax = (int64_t)a.pos0 + a.q_base + a.n_q;       // keys of the slice's last query
+  const int units = a.nkv * a.nqb;
+  const int64_t mxmost = (int64_t)kPvSplit * kPxSlice * a.nh * kHd / ((int64_t)units * kPxRows);   // a.mx's space
+  // Scores. q8_0: one 8-wave workgroup per CU (its operand tiles fill the LDS); a 64-key tile takes it
+  // 2.0 us, the digits and the last stores 7 (512 queries onto 8192 keys: 137 us in one round of 256
+  // workgroups, 149 in two, 160 in four; 48 onto 6000: 29 in one, 46 in four). Units a workgroup takes:
+  // four where there are that many, so that each tile is converted for all of them.
+  if (kf == BKV_Q8_0) {
+    const int uq = a.nqb >= 3 ? 4 : a.nqb, tile = uq == 1 ? 2 * kPxTile : kPxTile;
+    const int items = a.nkv * ((a.nqb + uq - 1) / uq);
+    a.ksplit = px_ranges(items, (kmax + tile - 1) / tile, 256, 2000, 7000, 0, mxmost);
+    const dim3 grid(items * a.ksplit);
+#define BKV_LAUNCH_SCORE(UQ)                                                                             \
+  do {                                                                                                   \
+    if (pg) hipLaunchKernelGGL((prefill_score_q8_kernel<UQ, true>), grid, dim3(512), 0, st, a);          \
+    else hipLaunchKernelGGL((prefill_score_q8_kernel<UQ, false>), grid, dim3(512), 0, st, a);            \
+  } while (0)
+    if (uq == 4) BKV_LAUNCH_SCORE(4);
+    else if (uq == 2) BKV_LAUNCH_SCORE(2);
+    else BKV_LAUNCH_SCORE(1);
+#undef BKV_LAUNCH_SCORE
+  } else {
+    // fp16: 4-wave workgroups of two units (one: a chunk of up to 4 queries), four resident per CU sharing
+    // its matrix cores: 24 us for a 256-key tile of each. (300 queries onto 2000 keys: 67 us with every
+    // tile a workgroup, 1000 onto none: 75 us, 82-84 with fewer workgroups; 512 onto 8192: 352 us, 392
+    // with one unit and two sets of keys per wave.)
+    const int items = a.nkv * ((a.nqb + 1) / 2);
+    a.ksplit = px_ranges(items, (kmax + kPxTile16 - 1) / kPxTile16, 1024, 24000, 2000, 0, mxmost);
+    const dim3 grid(items * a.ksplit);
+    if (a.nqb == 1) {
+      if (pg) hipLaunchKernelGGL((prefill_score_f16_kernel<1, true>), grid, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL((prefill_score_f16_kernel<1, false>), grid, dim3(256), 0, st, a);
+    } else {
+      if (pg) hipLaunchKernelGGL((prefill_score_f16_kernel<2, true>), grid, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL((prefill_score_f16_kernel<2, false>), grid, dim3(256), 0, st, a);
+    }
+  }
+  // Sums. Up to one unit per CU: 7 exp waves keep up with the chain (48 queries onto 6000 keys: 36 us);
+  // more units: 3 exp waves each, several workgroups per CU (512 onto 8192: 127 against 134 us; 300 onto
+  // 2000: 30 against 37).
+  if (units <= 256) hipLaunchKernelGGL(prefill_sum_kernel<8>, dim3(units), dim3(512), 0, st, a);
+  else hipLaunchKernelGGL(prefill_sum_kernel<4>, dim3(units), dim3(256), 0, st, a);
+  // PV: one workgroup per CU, 3 us per tile and 8 for the rest (512 onto 8192: 104 us in one round; 48
+  // onto 6000: 17 us in one round, 28 in two)
+  const int items = a.nkv * ((a.n_q + kPvQ - 1) / kPvQ);
+  // (the merge reads a range's partials at about 4 TB/s)
+  a.pv_split = px_ranges(items, (kmax + kPfTile - 1) / kPfTile, 256, 3000, 8000, (int64_t)a.n_q * a.nh * kHd * 4 / 4000,
+                         kPvSplit * kPxSlice / a.n_q);
+  const dim3 pgrid(items * a.pv_split);
+  if (vf == BKV_Q8_0) {
+    if (pg) hipLaunchKernelGGL((prefill_pv64_kernel<1, true>), pgrid, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((prefill_pv64_kernel<1, false>), pgrid, dim3(512), 0, st, a);
+  } else {
+    if (pg) hipLaunchKernelGGL((prefill_pv64_kernel<0, true>), pgrid, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((prefill_pv64_kernel<0, false>), pgrid, dim3(512), 0, st, a);
+  }
+  if (a.pv_split == 1) return hipGetLastError();
+  const size_t n4 = (size_t)a.n_q * a.nh * (kHd / 4);
+  hipLaunchKernelGGL(prefill_pv_merge_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 

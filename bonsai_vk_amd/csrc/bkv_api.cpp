@@ -206,6 +206,12 @@ static int choose_path(const DecodePlan &p) {
   return kPathSplit;
 }
 
+// Contexts a decode takes in one workgroup per KV group (bkv_short.hip). q8_0 V, one layer of 8 in us
+// against the stream kernel: 6.7 / 16.9 at 1 key, 9.3 / 17.0 at 128, 13.2 / 17.3 at 256, 16.5 / 17.5 at
+// 400, 19.8 / 17.7 at 511 (the eighth V tile waits for a buffer); with fp16 K 18.8 / 19.5 at 400, 22.0 /
+// 19.6 at 511. fp16 V against the resident kernel: 9.1 / 23.3 at 64, 14.2 / 22.4 at 256, 21.9 / 22.5 at 511.
+static int short_decode_keys(int vfmt) { return vfmt == BKV_Q8_0 ? 448 : kShortKeys; }
+
 static bool aligned16(const void *p) { return p && ((uintptr_t)p & 15u) == 0; }
 
 static uint64_t slot_bytes(const bkv_cache_desc *d, int which) {
@@ -300,6 +306,18 @@ static int decode_common(const bkv_cache_desc *d, int layer, uint32_t nfill, con
   L.base = kstart;
 
   const int path = choose_path(p);
+  if (forced_path() < 0 && path != kPathSplit && nfill <= (uint32_t)short_decode_keys(d->v_fmt)) {
+    // the single launch of a short context: one workgroup per KV group
+    ShortArgs sa{};
+    sa.L = L; sa.nkv = d->nkv; sa.nh = d->nh; sa.pos0 = nfill - 1; sa.n_q = 1; sa.scale = d->scale;
+    sa.q = q; sa.qs = qs; sa.gate = gate; sa.gs = gs; sa.out = out; sa.out_gated = out_gated;
+    if (fused) sa.ap = *fused;
+    sa.e = keep_intermediates() ? (float *)(w + p.r_e) : nullptr;
+    sa.ld = p.ld;
+    sa.sum = (float *)(w + p.r_sum);
+    sa.status = (unsigned *)(w + p.r_status);
+    return hip_fail(launch_short(sa, d->k_fmt, d->v_fmt, st));
+  }
   if (path == kPathResident || path == kPathStream) {
     ResArgs ra{};
     ra.L = L; ra.nkv = d->nkv; ra.nh = d->nh; ra.nfill = nfill; ra.scale = d->scale;
@@ -494,6 +512,17 @@ static int prefill_common(const bkv_cache_desc *d, int layer, uint32_t pos0, int
   if (!workspace) return BKV_EWORKSPACE;
   if (((uintptr_t)workspace & 255u) != 0) return BKV_EALIGN;
   const size_t base = prefill_base(d);
+  if (!prefill_mfma_requested() && n_q > 1 && (int64_t)pos0 + n_q <= kShortKeys) {
+    // a short context: one launch, 4 queries per workgroup (the workspace is asked for all the same, so
+    // that a caller meets its size at the first chunk and not at a later one)
+    const size_t need = n_q >= kPxMinQ ? px_layout(d->nh, d->nkv, (int64_t)pos0 + n_q, kPxSlice, base).total
+                                       : plan_decode(d->nh, d->nkv, d->k_fmt, d->v_fmt, (int64_t)pos0 + n_q, d->page_tokens).total;
+    if (ws_bytes < need) return BKV_EWORKSPACE;
+    ShortArgs a{};
+    a.L = view(d, layer); a.nkv = d->nkv; a.nh = d->nh; a.pos0 = pos0; a.n_q = n_q; a.scale = d->scale;
+    a.q = q; a.qs = qs; a.gate = gate; a.gs = gs; a.out = out; a.out_gated = out_gated;
+    return hip_fail(launch_short(a, d->k_fmt, d->v_fmt, stream));
+  }
   if (!prefill_mfma_requested() && n_q >= kPxMinQ) {
     // the exact kernels, in equal slices (of kPxSlice queries in a workspace without room for more)
     const int64_t ctx = (int64_t)pos0 + n_q;

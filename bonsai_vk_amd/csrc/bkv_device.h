@@ -18,9 +18,13 @@ __device__ __forceinline__ uint32_t lds_addr(const void *p) {
 // One 32-lane half wave writes one head row. q8_0: lanes 0..15 each own 16 consecutive elements
 // (half a block); the block absmax pairs lanes 2k and 2k+1. fp16: all 32 lanes own 8 elements.
 // (attn_norm_rope2.comp:167-217 for the arithmetic; the lane mapping is this kernel's own.)
+struct PackedRow {
+  uint4 d;                       // the lane's 16 bytes of data (q8_0: lanes 0..15)
+  uint32_t s;                    // q8_0, lanes 0, 4, 8, 12: two block scales
+};
 template <int FMT, bool RHAZ>
-__device__ __forceinline__ void append_row(const float *__restrict__ x, uint8_t *__restrict__ drow,
-                                           uint8_t *__restrict__ srow, int sub) {
+__device__ __forceinline__ PackedRow pack_row(const float *__restrict__ x, int sub) {
+  PackedRow r;
   if (FMT == BKV_Q8_0) {
     const int s = sub & 15;
     const float4 *xp = reinterpret_cast<const float4 *>(x + 16 * s);
@@ -42,19 +46,32 @@ __device__ __forceinline__ void append_row(const float *__restrict__ x, uint8_t 
              (q8_byte<RHAZ>(v[4 * i + 2], id) << 16) | (q8_byte<RHAZ>(v[4 * i + 3], id) << 24);
     const uint32_t h = f32_to_f16_rne(q8_scale(amax));
     const uint32_t hn = __shfl_down(h, 2);       // scale of the next block (lane s+2)
-    if (sub < 16) {
-      *reinterpret_cast<uint4 *>(drow + 16 * s) = make_uint4(w[0], w[1], w[2], w[3]);
-      if ((s & 3) == 0) *reinterpret_cast<uint32_t *>(srow + (s >> 2) * 4) = h | (hn << 16);
-    }
+    r.d = make_uint4(w[0], w[1], w[2], w[3]);
+    r.s = h | (hn << 16);
   } else {
     const float4 *xp = reinterpret_cast<const float4 *>(x + 8 * sub);
     const float4 a = xp[0], b = xp[1];
-    const uint4 o = make_uint4(f32_to_f16_rne(a.x) | (f32_to_f16_rne(a.y) << 16),
-                               f32_to_f16_rne(a.z) | (f32_to_f16_rne(a.w) << 16),
-                               f32_to_f16_rne(b.x) | (f32_to_f16_rne(b.y) << 16),
-                               f32_to_f16_rne(b.z) | (f32_to_f16_rne(b.w) << 16));
-    *reinterpret_cast<uint4 *>(drow + 16 * sub) = o;
+    r.d = make_uint4(f32_to_f16_rne(a.x) | (f32_to_f16_rne(a.y) << 16), f32_to_f16_rne(a.z) | (f32_to_f16_rne(a.w) << 16),
+                     f32_to_f16_rne(b.x) | (f32_to_f16_rne(b.y) << 16), f32_to_f16_rne(b.z) | (f32_to_f16_rne(b.w) << 16));
+    r.s = 0;
   }
+  return r;
+}
+template <int FMT>
+__device__ __forceinline__ void store_row(const PackedRow &r, uint8_t *__restrict__ drow, uint8_t *__restrict__ srow, int sub) {
+  if (FMT == BKV_Q8_0) {
+    if (sub < 16) {
+      *reinterpret_cast<uint4 *>(drow + 16 * sub) = r.d;
+      if ((sub & 3) == 0) *reinterpret_cast<uint32_t *>(srow + sub) = r.s;
+    }
+  } else {
+    *reinterpret_cast<uint4 *>(drow + 16 * sub) = r.d;
+  }
+}
+template <int FMT, bool RHAZ>
+__device__ __forceinline__ void append_row(const float *__restrict__ x, uint8_t *__restrict__ drow,
+                                           uint8_t *__restrict__ srow, int sub) {
+  store_row<FMT>(pack_row<FMT, RHAZ>(x, sub), drow, srow, sub);
 }
 
 // one wave: lanes 0..31 write the K row, lanes 32..63 the V row of (token t, head g)

@@ -131,6 +131,26 @@ struct ResArgs {
   unsigned *tsw;                 // per-wave phase timestamps [workgroup][8 waves][8] (experiment builds)
 };
 
+// ------------------------------------------------------------------ short contexts, one workgroup per row group
+constexpr int kShortKeys = 512;  // keys a workgroup holds
+
+struct ShortArgs {
+  LayerView L;
+  int nkv, nh;
+  uint32_t pos0;                 // query i attends over keys 0 .. pos0 + i (pos0 + n_q <= kShortKeys)
+  int n_q;
+  float scale;
+  const float *q, *gate;         // [n_q][nh] rows, qs / gs floats apart
+  int qs, gs;
+  float *out, *out_gated;
+  AppendArgs ap;                 // decode_step (n_q 1): the token to append, key pos0 (ap.k null: none)
+  float *e;                      // n_q 1: [nh][ld] when kept (diagnostics), or null
+  int64_t ld;
+  float *sum;                    // n_q 1: [nh]
+  unsigned *status;              // n_q 1: [nh]
+};
+hipError_t launch_short(const ShortArgs &a, int kf, int vf, hipStream_t st);
+
 // ------------------------------------------------------------------ chunked prefill (MFMA)
 constexpr int kPfQ = 16;       // queries per workgroup (x 4 heads = 64 rows)
 constexpr int kPfTile = 64;    // keys per tile

@@ -28,56 +28,13 @@
 #include "bkv_device.h"
 #include "bkv_exp.h"
 #include "bkv_internal.h"
+#include "bkv_mfma16.h"
 #include "bkv_pv8.h"
 
 namespace bkv {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef short v4s_t __attribute__((ext_vector_type(4)));
-typedef short v8s_t __attribute__((ext_vector_type(8)));
-
 constexpr int kPfNT = 256;      // 4 waves
 constexpr int kPfRS = 144;      // LDS row stride in bytes of the P and V^T tiles (64 fp16 + pad)
-
-__device__ __forceinline__ f4 mfma16(h8 a, h8 b, f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ h2 as_h2(uint32_t w) { return __builtin_bit_cast(h2, w); }
-__device__ __forceinline__ uint32_t as_u(h2 v) { return __builtin_bit_cast(uint32_t, v); }
-
-// two signed bytes of w (already biased by 0x80 per byte), selected by SEL, as an exact fp16 pair:
-// 0x64XX is the fp16 number 1024 + XX, so subtracting 1152 leaves the signed byte value.
-template <uint32_t SEL>
-__device__ __forceinline__ h2 bytes_h2(uint32_t wb) {
-  const h2 x = as_h2(__builtin_amdgcn_perm(0x64646464u, wb, SEL));
-  return x - h2{(_Float16)1152.0f, (_Float16)1152.0f};
-}
-
-// e / s correctly rounded to fp32, from rs = fp32(1/s) correctly rounded, without a division:
-// q0 = e*rs is within 1.5 ulps of e/s; one correction q1 = q0 + (e - s*q0)*rs (the remainder exact
-// by fma) brings it within one ulp, and a second is then the correctly rounded quotient (Markstein's
-// theorem: y within half an ulp of 1/s, q within one ulp of e/s, r = e - s*q exact => RN(q + r*y)
-// = RN(e/s)). Valid for 0 <= e <= s, s >= 1 (a softmax sum includes the maximum's e = 1): the
-// remainders stay normal while the quotient is above 2^-60, and below that the quotient rounds to
-// an fp16 zero whatever its last bits.
-__device__ __forceinline__ float div_by_sum(float e, float s, float rs) {
-  const float q0 = e * rs;
-  const float q1 = __builtin_fmaf(__builtin_fmaf(-s, q0, e), rs, q0);
-  float q2 = __builtin_fmaf(__builtin_fmaf(-s, q1, e), rs, q1);
-  // the fp32 result itself: a conversion to fp16 of the fma would otherwise be folded into one
-  // mixed-precision fma rounding once, straight to fp16 (a different result at fp16 ties)
-  asm volatile("" : "+v"(q2));
-  return q2;
-}
-
-// exact fp16 split of s*b: hi = f16(s*b) (rounded fp16 product), lo = the product's rounding error
-__device__ __forceinline__ void split_prod(h2 b, h2 s, h2 &hi, h2 &lo) {
-  hi = b * s;
-  lo = __builtin_elementwise_fma(b, s, -hi);
-}
 
 // exp(x) for x <= 0 (or -inf) in fp32 to about 2 ulp: 2^(x log2 e) on the hardware exp2 with the
 // rounding error of the product x*log2(e) carried as a first-order correction
@@ -511,14 +468,6 @@ hipError_t launch_prefill(const PrefillArgs &a, int kf, int vf, hipStream_t st) 
 //   merge   the key ranges' partials added in order, and the gate.
 // Only the PV sum runs in another order than the reference (fp32 accumulation of exact products).
 
-// Workgroup barrier for LDS traffic only: every wave's LDS operations have completed, while its
-// global loads (prefetches a step or more ahead) stay in flight. __syncthreads() also releases
-// global memory, i.e. waits for every outstanding load and store of the wave first, which would
-// void those prefetches. Used where the waves exchange data through LDS alone.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 // scratch accesses (plain loads and stores: the scratch round trips are served largely by the
 // memory-side cache, which non-temporal accesses bypass)
 __device__ __forceinline__ void st_sc4(float *p, float4 v) { *reinterpret_cast<float4 *>(p) = v; }
@@ -552,96 +501,6 @@ __device__ __forceinline__ PxItem px_item(const PrefillXArgs &a) {
   return p;
 }
 
-// ---------------------------------------------------------------- q8_0 K scores on the matrix cores
-// The contract's inner sum (bkv_q8dot.h) is the fp32 rounding of the exact sum of q16 * int8 over a
-// block. fp16 MFMAs give it with two digits per q16, q = hi + lo: hi a multiple of u and lo a multiple
-// of t, where u is the smallest power of two with sum |hi| * 128 <= 2^24 u in every block of the row, and
-// sum |lo| * 128 <= 2^24 t. All products of a digit with bytes in [-128, 127] and all their partial sums
-// are then multiples of the digit's unit below 2^24 units: the MFMA's fp32 sums are exact in any
-// order, and fp32(hi sum + lo sum) is one fma with one rounding (lo is kept scaled by 2^8): one VALU
-// instruction per block and score, where int8 digits need two shifted adds, two conversions, an fma in
-// fp64 and its rounding. The row is scaled by a power of two so that u = 2^-2: hi <= 2^15, lo * 2^8 <= 2^5
-// in units above 2^-14, all fp16 normals; hi has at most 11 significant bits (a q16 of 2^10 u or more is
-// itself a multiple of u), lo at most 11 (it is q16 or a remainder of it).
-// A block whose lo is no multiple of such a t in some row (a q16 about 2^-16 of the row's largest or
-// less: one of a hundred rows of normal values has one) gets a third digit: lo a multiple of 2^-13 u,
-// lo2 = the rest, a multiple of 2^-26 u, kept scaled by 2^14. It costs a third MFMA, and its three sums
-// are combined in fp64 (below 2^53 units: exact) and rounded once. Rows that need more, or hold Inf / NaN,
-// take the fp64 VALU path.
-constexpr int kDigUnit = 2 * 8 * 64;               // 16-byte operands per unit: [pair j][block][lane]
-
-// Cooperative (256 threads, tid their index): the A operands of a unit's q rows (rows(i): the 4 head
-// rows of query i) in dig [pair][block][lane] (pair j: rows 4 i + 2 (h % 2) + digit for heads h = 2 j,
-// 2 j + 1 of query i) and lo2 [block][lane] (rows 4 i + h); lane l of an operand holds row l % 16, dims
-// 8 (l/16) .. + 7 of the block. ex[row 4 i + h]: the score's power of two. *flags: bit b set when block b
-// of any row has a third digit; *wide when the rows need the fp64 path. Both zeroed by the caller.
-template <typename ROWS>
-__device__ __forceinline__ void px_digits(int tid, const ROWS &rows, int qs, uint4 *dig, uint4 *lo2, float *ex,
-                                          unsigned *flags, unsigned *wide) {
-  const int r = tid >> 4, p = tid & 15, qi = r >> 2, h = r & 3;
-  const float *src = rows(qi) + (size_t)h * qs + 16 * p;
-  float x[16], s = 0.0f;
-  bool bad = false;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float4 t = *reinterpret_cast<const float4 *>(src + 4 * i);
-    x[4 * i] = round_f16(t.x); x[4 * i + 1] = round_f16(t.y);
-    x[4 * i + 2] = round_f16(t.z); x[4 * i + 3] = round_f16(t.w);
-  }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    bad = bad || !(fabsf(x[i]) <= 65504.0f);
-    s += fabsf(x[i]);
-  }
-  s += dpp<0xB1>(s);                               // the block's (two lanes hold one)
-  s = row16_max(s);                                // the row's largest
-  // S = s below 2^(E+1) (below 0.999 of it, for s's rounding and the u/2 that rounding adds to each hi):
-  // u = 2^(E-16); scaled so that u = 2^-2
-  const uint32_t sb = __float_as_uint(s);
-  const int E = s > 0.0f ? (int)(sb >> 23) - 127 + ((sb & 0x7FFFFFu) > 0x7FBFFFu ? 1 : 0) : 14;
-  bad = bad || E > 100;                            // (Inf / NaN rows: any finite scale)
-  const float up = bad ? 1.0f : __uint_as_float((uint32_t)(127 + 14 - E) << 23);
-  float lr[16], L = 0.0f;
-  h8 d0[2], d1[2], d2[2];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const float y = x[i] * up;                     // exact
-    const float hi = __builtin_rintf(y * 4.0f) * 0.25f;
-    lr[i] = y - hi;                                // exact, at most 2^-3
-    L += fabsf(lr[i]);
-    d0[i >> 3][i & 7] = (_Float16)hi;
-  }
-  L += dpp<0xB1>(L);
-  // t = 2^(exponent of L + 1 - 17), at least 2^-22: L * 128 < 2^24 t (L's fp32 rounding is far below the
-  // factor of up to 2 that the exponent leaves, except where L is within 2^-18 of a power of two: + 1)
-  const uint32_t lb = __float_as_uint(L) + 64u;
-  const float ti = __uint_as_float((uint32_t)(254 - max((int)(lb >> 23) + 1 - 17, 127 - 22)) << 23);   // 1 / t
-  bool fine = true;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) fine = fine && __builtin_rintf(lr[i] * ti) == lr[i] * ti;
-  const bool third = !(fine && dpp<0xB1>(fine ? 1.0f : 0.0f) == 1.0f);
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const float lo = third ? __builtin_rintf(lr[i] * 32768.0f) * 0x1p-15f : lr[i];
-    const float l2 = (lr[i] - lo) * 16384.0f;      // exact, at most 2^-2
-    bad = bad || __builtin_rintf(l2 * 16384.0f) != l2 * 16384.0f;
-    d1[i >> 3][i & 7] = (_Float16)(lo * 256.0f);
-    d2[i >> 3][i & 7] = (_Float16)l2;
-  }
-  const int b = p >> 1;
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int lq = 2 * (p & 1) + k, l = 16 * lq + 4 * qi + 2 * (h & 1);
-    uint4 *o = dig + ((h >> 1) * 8 + b) * 64;
-    o[l] = __builtin_bit_cast(uint4, d0[k]);
-    o[l + 1] = __builtin_bit_cast(uint4, d1[k]);
-    lo2[b * 64 + 16 * lq + r] = __builtin_bit_cast(uint4, d2[k]);
-  }
-  if (p == 0) ex[r] = 1.0f / up;
-  if (third) atomicOr(flags, 1u << b);
-  if (bad) atomicOr(wide, 1u);
-}
-
 // A workgroup scores UQ units against its range of key tiles (TILE keys each; UQ = 1: 128, else 64).
 // The tile's bytes become fp16 B operands in LDS once for all its units (2.5 instructions per 4 bytes:
 // at one unit per conversion they were a third of the kernel's VALU work), a tile ahead of the MFMAs:
@@ -654,13 +513,13 @@ __global__ __launch_bounds__(512, 1) void prefill_score_q8_kernel(PrefillXArgs a
   const PxItem p = px_item<UQ, TILE>(a);
   const int tid = threadIdx.x, lane = tid & 63, ql = lane >> 4, n16 = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), u = w % UQ, kg0 = NKG * (w / UQ);
-  __shared__ uint4 s_op[2][KGS * 8 * 64];          // first the units' digits (kDigUnit each), then the tiles
+  __shared__ uint4 s_op[2][KGS * 8 * 64];          // first the units' digits (kQ8fUnit each), then the tiles
   __shared__ __attribute__((aligned(16))) float s_sc[2][TILE][8];
   __shared__ uint4 s_lo2[UQ][8 * 64];
   __shared__ float s_ex[UQ][kPxRows];
   __shared__ float s_red[8][kPxRows];
   __shared__ unsigned s_flags[UQ], s_wide;
-  static_assert(sizeof(s_op) >= UQ * kDigUnit * 16, "the units' digits in the operand buffers");
+  static_assert(sizeof(s_op) >= UQ * kQ8fUnit * 16, "the units' digits in the operand buffers");
   uint4 *const op = &s_op[0][0];
   if (tid < UQ) s_flags[tid] = 0u;
   if (tid == 0) s_wide = 0u;
@@ -673,15 +532,16 @@ __global__ __launch_bounds__(512, 1) void prefill_score_q8_kernel(PrefillXArgs a
   };
   for (int i = tid >> 8; i < UQ; i += 2) {
     const int q0 = a.q_base + kPxQ * unit(i);
-    px_digits(tid & 255, [&](int q) { return qrows(q0 + q); }, a.qs, op + i * kDigUnit, s_lo2[i], s_ex[i], &s_flags[i],
-              &s_wide);
+    Q8fRaw raw;
+    q8f_fetch(tid & 255, [&](int q) { return qrows(q0 + q); }, a.qs, raw);
+    q8f_digits(tid & 255, raw, op + i * kQ8fUnit, s_lo2[i], s_ex[i], &s_flags[i], &s_wide);
   }
   __syncthreads();
   h8 da[2][8];                                     // the A operands of the wave's unit
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int b = 0; b < 8; ++b) da[j][b] = __builtin_bit_cast(h8, op[u * kDigUnit + (j * 8 + b) * 64 + lane]);
+    for (int b = 0; b < 8; ++b) da[j][b] = __builtin_bit_cast(h8, op[u * kQ8fUnit + (j * 8 + b) * 64 + lane]);
   const int uq = kPxQ * unit(u) + ql;              // the lane's query in the slice
   const int lim = uq < a.n_q ? (int)(a.pos0 + (uint32_t)(a.q_base + uq)) : -1;   // the last key it sees
   const unsigned flags = (unsigned)__builtin_amdgcn_readfirstlane((int)s_flags[u]);
@@ -831,16 +691,6 @@ __global__ __launch_bounds__(512, 1) void prefill_score_q8_kernel(PrefillXArgs a
 // holds D_b[4(l/16) + k][l%16] in accumulator register 4b + k. With K = 1 each step is exactly one
 // fp32 fma per element (the product of two fp16 values is exact in fp32), so a chain of steps in
 // ascending dimension is the reference's serial score, bit for bit. (q8_0 K: bkv_q8dot.h.)
-typedef float fv16 __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ fv16 mfma_k1(float a, float b, fv16 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ uint32_t word_of(const uint4 &v, int i) {
-  return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-}
-
 // A workgroup scores NU units against its range of 256-key tiles: one chain of 256 steps per (row,
 // key), acc = acc + q16*k in ascending dimension. Block b of the instruction is key group b (keys 16b ..
 // + 15 of the wave's 64), so one MFMA advances 64 keys x 16 rows; the wave's NU units are independent

@@ -90,11 +90,15 @@ __device__ __forceinline__ void q8lim_build(const float *q, int qs, int8_t *lim,
   }
 }
 
-__device__ __forceinline__ void q8lim_load(const int8_t *lim, const int *lt, Q8Lim &L) {
-  const int lane = threadIdx.x & 63, m = lane & 15, kq = lane >> 4;
+// (pq: the lane takes dims 8 pq .. + 7 of each block, for B operands in another order than lane / 16)
+__device__ __forceinline__ void q8lim_load(const int8_t *lim, const int *lt, Q8Lim &L, int pq) {
+  const int lane = threadIdx.x & 63, m = lane & 15;
 #pragma unroll
-  for (int b = 0; b < 8; ++b) L.a[b] = *reinterpret_cast<const long *>(lim + (b * 16 + m) * 32 + 8 * kq);
-  L.t = lt[kq];
+  for (int b = 0; b < 8; ++b) L.a[b] = *reinterpret_cast<const long *>(lim + (b * 16 + m) * 32 + 8 * pq);
+  L.t = lt[lane >> 4];
+}
+__device__ __forceinline__ void q8lim_load(const int8_t *lim, const int *lt, Q8Lim &L) {
+  q8lim_load(lim, lt, L, (threadIdx.x & 63) >> 4);
 }
 
 __device__ __forceinline__ float f16_half(uint32_t w, int hi) { return f16_to_f32(hi ? (w >> 16) : (w & 0xFFFFu)); }

@@ -43,8 +43,8 @@ def queries(n, kind):
 
 # edges of the 64-key tiles, of the 64/128/256-query groups, one to four and more units, several key ranges
 @pytest.mark.parametrize("kf,vf,pos0,n,kind", [
-    (BKV_Q8_0, BKV_Q8_0, 0, 16, "normal"), (BKV_Q8_0, BKV_Q8_0, 47, 17, "normal"),
-    (BKV_Q8_0, BKV_Q8_0, 300, 33, "normal"), (BKV_Q8_0, BKV_F16, 3000, 40, "third"),
+    (BKV_Q8_0, BKV_Q8_0, 560, 16, "normal"), (BKV_Q8_0, BKV_Q8_0, 687, 17, "normal"),
+    (BKV_Q8_0, BKV_Q8_0, 940, 33, "normal"), (BKV_Q8_0, BKV_F16, 3000, 40, "third"),
     (BKV_Q8_0, BKV_Q8_0, 1000, 20, "wide"), (BKV_Q8_0, BKV_Q8_0, 700, 19, "tiny"),
     (BKV_Q8_0, BKV_Q8_0, 640, 18, "mixed"), (BKV_Q8_0, BKV_Q8_0, 2000, 513, "normal"),
     (BKV_Q8_0, BKV_Q8_0, 8000, 521, "normal"), (BKV_F16, BKV_Q8_0, 900, 21, "normal"),

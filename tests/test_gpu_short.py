@@ -1,0 +1,100 @@
+"""GPU: the single launch of contexts of at most 512 keys (one workgroup per KV group) against the stream,
+resident and chunk kernels, which the other tests hold to the oracle: scores' e, sums and cache bytes bit
+for bit, outputs to the fp32 order of the PV sum (each a sum of at most 512 exact products of magnitude
+below the row's largest |v|: 512 * 2^-24 of it bounds the difference of two orders)."""
+import pytest
+import torch
+
+import oracle
+from bonsai_vk_amd import BKV_F16, BKV_Q8_0, KvCache
+from tests.gpu_util import say
+
+pytestmark = pytest.mark.gpu
+FMTS = [(BKV_Q8_0, BKV_Q8_0), (BKV_F16, BKV_F16), (BKV_F16, BKV_Q8_0), (BKV_Q8_0, BKV_F16)]
+TOL = 512 * 2.0 ** -24
+
+
+def caches(n, kf, vf, page):
+    kw = {}
+    cap = n
+    if page:
+        pool = -(-n // page) + 3
+        kw = {"page_tokens": page, "max_pages": pool, "block_table": torch.randperm(pool, generator=torch.Generator().manual_seed(n))[None]}
+        cap = pool * page
+    out = []
+    k, v = oracle.synth_kv(n, 4, 256, 3, 0, outliers=3)
+    k, v = torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda()
+    for _ in range(2):
+        c = KvCache(n_layers=1, cap=cap, k_fmt=kf, v_fmt=vf, max_ctx=n, **kw)
+        if n > 1:
+            c.append(0, 0, k[:n - 1], v[:n - 1])
+        out.append(c)
+    return out[0], out[1], k, v
+
+
+def queries(n, kind):
+    q = torch.from_numpy(oracle.normal(n * 16 * 256, 5, 3).reshape(n, 16, 256).copy())
+    if kind == "wide":                             # the fp64 path of the q8_0 scores
+        q[..., 5] *= 300
+        q[..., 70] = 1e-6
+    if kind == "third":                            # blocks with three digits
+        q[..., ::8] *= 1e-4
+    return q.cuda()
+
+
+def same_caches(a, b):
+    return all(x is None or torch.equal(x, y) for x, y in zip(a.host_arrays(), b.host_arrays()))
+
+
+# edges: 16-key groups, 64-key tiles, 128-key rounds, three and more V tiles, the limit
+@pytest.mark.parametrize("kf,vf", FMTS)
+@pytest.mark.parametrize("n,page", [(1, 0), (2, 64), (16, 0), (64, 0), (65, 64), (129, 0), (192, 0), (257, 128), (300, 0),
+                                    (449, 64), (512, 0)])
+def test_short_decode(kf, vf, n, page, monkeypatch):
+    say(f"short decode kf={kf} vf={vf} n={n} page={page}")
+    monkeypatch.setenv("BKV_KEEP_INTERMEDIATES", "1")
+    a, b, k, v = caches(n, kf, vf, page)
+    q = queries(1, "wide" if n == 129 else "normal")[0]
+    gate = queries(1, "normal")[0].flip(0).contiguous()
+    args = (0, n - 1, k[n - 1:], v[n - 1:], q, gate)
+    out, og = a.decode_step(*args)
+    torch.cuda.synchronize()
+    _, e, s, st = a.debug_intermediates(n)
+    monkeypatch.setenv("BKV_DECODE", "stream")     # (fp16 V: the resident kernel)
+    want, wg = b.decode_step(*args)
+    torch.cuda.synchronize()
+    _, e2, s2, _ = b.debug_intermediates(n)
+    assert torch.equal(e, e2) and torch.equal(s, s2) and int(st.abs().sum()) == 0
+    assert same_caches(a, b)
+    tol = TOL * float(v.abs().max())
+    assert float((out - want).abs().max()) <= tol and float((og - wg).abs().max()) <= tol
+    # the same from a window that starts inside a page and a tile, and from interleaved q / gate rows
+    if n > 40:
+        wb, _ = b.decode_window(0, 37, n, q)
+        monkeypatch.delenv("BKV_DECODE")
+        wa, _ = a.decode_window(0, 37, n, q)
+        qg = torch.stack([q, gate], 1).reshape(16, 512).contiguous()
+        oq, ogq = a.decode_qg(0, n, qg)
+        torch.cuda.synchronize()
+        assert float((wa - wb).abs().max()) <= tol
+        assert torch.equal(oq, out) and torch.equal(ogq, og)
+
+
+@pytest.mark.parametrize("kf,vf", FMTS)
+@pytest.mark.parametrize("pos0,n,page,kind", [(0, 2, 0, "normal"), (0, 5, 64, "normal"), (60, 9, 0, "third"), (100, 30, 0, "wide"),
+                                              (0, 131, 0, "normal"), (300, 77, 64, "normal"), (495, 17, 0, "third"), (0, 512, 0, "normal")])
+def test_short_prefill(kf, vf, pos0, n, page, kind, monkeypatch):
+    """Each row of a chunk against the stream or resident decode of the same query."""
+    say(f"short prefill kf={kf} vf={vf} pos0={pos0} n={n} page={page} {kind}")
+    a, _, k, v = caches(pos0 + n, kf, vf, page)
+    a.append(0, pos0 + n - 1, k[-1:], v[-1:])
+    q = queries(n, kind)
+    gate = queries(n, "normal").flip(1).contiguous()
+    out, og = a.prefill_chunk(0, pos0, q, gate)
+    monkeypatch.setenv("BKV_DECODE", "stream")
+    tol = TOL * float(v.abs().max())
+    for i in sorted({0, 1, 2, 3, 4, n // 2, n - 2, n - 1} & set(range(n))):
+        want, wg = a.decode(0, pos0 + i + 1, q[i].contiguous(), gate[i].contiguous())
+        torch.cuda.synchronize()
+        assert float((out[i] - want).abs().max()) <= tol, i
+        assert float((og[i] - wg).abs().max()) <= tol, i

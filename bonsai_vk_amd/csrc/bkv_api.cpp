@@ -496,6 +496,14 @@ int bkv_decode_step_qg(const bkv_cache_desc *d, int layer, uint32_t pos, const f
                             workspace, ws_bytes, stream, 2 * kHd, 2 * kHd);
 }
 
+// Whether a chunk of 2 to kPxMinQ - 1 queries runs as one chunk (true) or as decode rows: the chunk takes
+// about 26 us and 6.2 ns per key of its last row (its serial sums) whatever its length, a decode row 17 us
+// and 0.4 ns per key. us for the attention, rows / chunk: 2 queries at 3000 keys 37 / 47, 3 at 3000 55 / 47,
+// 6 at 3000 110 / 49, 3 at 8000 61 / 73, 8 at 8000 160 / 73, 6 at 32000 168 / 228, 12 at 32000 335 / 212.
+static bool px_worthwhile(int n_q, int64_t keys) {
+  return n_q >= kPxMinQ || (n_q > 1 && n_q * (170000 + 4 * keys) > 260000 + 62 * keys);
+}
+
 static int prefill_common(const bkv_cache_desc *d, int layer, uint32_t pos0, int n_q,
                           const float *q, const float *gate, float *out, float *out_gated,
                           void *workspace, size_t ws_bytes, hipStream_t stream, int qs, int gs) {
@@ -523,7 +531,8 @@ static int prefill_common(const bkv_cache_desc *d, int layer, uint32_t pos0, int
     a.q = q; a.qs = qs; a.gate = gate; a.gs = gs; a.out = out; a.out_gated = out_gated;
     return hip_fail(launch_short(a, d->k_fmt, d->v_fmt, stream));
   }
-  if (!prefill_mfma_requested() && n_q >= kPxMinQ) {
+  if (!prefill_mfma_requested() && px_worthwhile(n_q, (int64_t)pos0 + n_q) &&
+      (n_q >= kPxMinQ || ws_bytes >= px_layout(d->nh, d->nkv, (int64_t)pos0 + n_q, kPxSlice, base).total)) {
     // the exact kernels, in equal slices (of kPxSlice queries in a workspace without room for more)
     const int64_t ctx = (int64_t)pos0 + n_q;
     if (ws_bytes < px_layout(d->nh, d->nkv, ctx, kPxSlice, base).total) return BKV_EWORKSPACE;
@@ -558,7 +567,7 @@ static int prefill_common(const bkv_cache_desc *d, int layer, uint32_t pos0, int
     return BKV_OK;
   }
   if (!prefill_mfma_requested()) {
-    // short chunks: every row is the decode row at nfill = pos0 + i + 1
+    // short chunks (also in a workspace for decodes only): every row is the decode row at nfill = pos0 + i + 1
     const size_t rs = (size_t)d->nh * d->hd;
     for (int i = 0; i < n_q; ++i) {
       rc = decode_common(d, layer, pos0 + (uint32_t)i + 1u, q + i * (size_t)d->nh * qs,

@@ -47,7 +47,8 @@ def queries(n, kind):
     (BKV_Q8_0, BKV_Q8_0, 940, 33, "normal"), (BKV_Q8_0, BKV_F16, 3000, 40, "third"),
     (BKV_Q8_0, BKV_Q8_0, 1000, 20, "wide"), (BKV_Q8_0, BKV_Q8_0, 700, 19, "tiny"),
     (BKV_Q8_0, BKV_Q8_0, 640, 18, "mixed"), (BKV_Q8_0, BKV_Q8_0, 2000, 513, "normal"),
-    (BKV_Q8_0, BKV_Q8_0, 8000, 521, "normal"), (BKV_F16, BKV_Q8_0, 900, 21, "normal"),
+    (BKV_Q8_0, BKV_Q8_0, 8000, 521, "normal"),
+    (BKV_Q8_0, BKV_Q8_0, 1400, 3, "normal"), (BKV_Q8_0, BKV_F16, 1400, 7, "third"), (BKV_F16, BKV_Q8_0, 2100, 4, "normal"), (BKV_F16, BKV_Q8_0, 900, 21, "normal"),
     (BKV_F16, BKV_F16, 495, 130, "normal"), (BKV_F16, BKV_Q8_0, 0, 600, "normal")])
 def test_prefill_e_and_sums_equal_decode(kf, vf, pos0, n, kind, monkeypatch):
     monkeypatch.setenv("BKV_KEEP_INTERMEDIATES", "1")
@@ -76,3 +77,21 @@ def test_prefill_e_and_sums_equal_decode(kf, vf, pos0, n, kind, monkeypatch):
         got = e[:, i // 4, i % 4, :nfill, :].permute(0, 2, 1).reshape(16, nfill).cpu()
         assert torch.equal(got, want), (i, int((got != want).sum()))
         assert torch.equal(sums[:, i // 4, i % 4, :].reshape(16).cpu(), s), i
+
+
+def test_small_chunk_in_a_decode_workspace():
+    """Chunks of 2 to 15 queries are accepted in a workspace sized for decodes (as decode rows), with the
+    results of the chunk in a prefill workspace up to the order of the PV sum."""
+    pos0, n = 1400, 5
+    cache = KvCache(n_layers=1, cap=pos0 + n, k_fmt=BKV_Q8_0, v_fmt=BKV_Q8_0)
+    k, v = oracle.synth_kv(pos0 + n, 4, 256, 7, 0, outliers=3)
+    cache.append(0, 0, torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda())
+    q = queries(n, "normal")
+    out, _ = cache.prefill_chunk(0, pos0, q)
+    want = torch.empty_like(out)
+    rc = lib().bkv_attn_prefill_chunk(ctypes.byref(cache.desc), 0, pos0, n, q.data_ptr(), None, want.data_ptr(), None,
+                                      cache.workspace.data_ptr(), cache.workspace.numel(), cache._stream())
+    torch.cuda.synchronize()
+    assert rc == 0
+    # (each output a sum of pos0 + n products with a probability sum of 1)
+    assert float((out - want).abs().max()) <= (pos0 + n) * 2.0 ** -24 * float(abs(v).max())

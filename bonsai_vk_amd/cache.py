@@ -96,6 +96,7 @@ class KvCache:
             return torch.zeros((n_layers, cap, row), dtype=torch.uint8, device=self.device)
 
         self.k_data = alloc(k_fmt, False)
+        self._dev = self.k_data.device             # (with its index, unlike self.device)
         self.k_scales = alloc(k_fmt, True)
         self.v_data = alloc(v_fmt, False)
         self.v_scales = alloc(v_fmt, True)
@@ -132,13 +133,17 @@ class KvCache:
         return None if t is None else t.data_ptr()
 
     def _f32(self, t, shape):
-        t = torch.as_tensor(t, dtype=torch.float32, device=self.device).contiguous()
-        assert tuple(t.shape) == tuple(shape), (tuple(t.shape), shape)
+        # a tensor that is as the call needs it is taken as it is (as_tensor and contiguous would return
+        # it too, 2 us later: a decode makes four such checks per layer)
+        if type(t) is not torch.Tensor or t.dtype is not torch.float32 or t.device != self._dev or not t.is_contiguous():
+            t = torch.as_tensor(t, dtype=torch.float32, device=self.device).contiguous()
+        assert t.shape == shape, (tuple(t.shape), shape)
         return t
 
     @staticmethod
     def _stream():
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        """The current stream of the current device, without a torch.cuda.Stream object around it."""
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
     # ---------------------------------------------------------------- the path
     def append(self, layer, pos, k, v):

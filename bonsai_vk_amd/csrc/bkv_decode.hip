@@ -12,7 +12,8 @@
 #include "bkv_common.h"
 #include "bkv_device.h"
 #include "bkv_internal.h"
-#include "bkv_q8dot.h"
+#include "bkv_mfma16.h"
+#include "bkv_pv8.h"
 
 namespace bkv {
 
@@ -22,58 +23,130 @@ __global__ __launch_bounds__(64) void append_kernel(AppendArgs a) {
   append_token<KF, VF, RHAZ>(a, (int64_t)a.pos + t, t, g, threadIdx.x);
 }
 
-template <int KF>
-struct QkTile {
-  static constexpr int DPR = KF == BKV_Q8_0 ? 16 : 32;      // data uint4 per K row
-  static constexpr int UPR = DPR + 1;                       // + scales / pad (bank spread)
-  static constexpr int NT = KF == BKV_Q8_0 ? 256 : 128;     // threads = keys per workgroup
-  static constexpr int KEYS = NT;
-};
+constexpr int kQkKeysQ8 = 256, kQkKeysF16 = 128;            // keys per workgroup
 
-template <int KF, int VF, bool FUSE, bool RHAZ>
-__global__ __launch_bounds__(QkTile<KF>::NT) void qk_kernel(QkArgs a) {
-  using T = QkTile<KF>;
-  constexpr int NT = T::NT;
-  __shared__ uint4 tile[T::KEYS * T::UPR];
+// q8_0 K: 4 waves x 64 keys, scored from registers. A wave requests its four groups of 16 keys in 16-byte
+// pieces (lane: key lane % 16, bytes 64 j + 16 (lane / 16) .. + 15, whose halves then change places between
+// lanes) behind the q rows (loads return in order), so the digits of q are ready when K lands; nothing but
+// the digits goes through LDS. Bound by the K stream: 200,000 keys x 4 groups in 52 us (104 with the tile
+// staged in LDS by 70 KiB workgroups, whose loads and scores did not overlap).
+template <int VF, bool FUSE, bool RHAZ>
+__global__ __launch_bounds__(kQkKeysQ8) void qk_q8_kernel(QkArgs a) {
+  constexpr int NT = kQkKeysQ8;
+  const int c = blockIdx.x, g = blockIdx.y, tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t j0 = (int64_t)c * NT;
+  const int n = (int)min((int64_t)NT, (int64_t)a.nfill - j0);
+  const LayerView &L = a.L;
+  __shared__ __attribute__((aligned(16))) int8_t s_lim[kLimBytes];
+  __shared__ __attribute__((aligned(16))) float s_q[kGqa][kHd];
+  __shared__ int s_lt[kGqa];
+  __shared__ unsigned s_wide;
+  __shared__ float s_max[4][kGqa], s_sum[4][kGqa];
+  const float *qg = a.q + (size_t)g * kGqa * a.qs;
+  const float4 q4 = reinterpret_cast<const float4 *>(qg + (size_t)w * a.qs)[lane];
+  if (tid == 0) s_wide = 0u;
+  if (c == 0 && g == 0 && tid < a.nkv * kGqa) a.counters[tid * kCounterStride] = 0u;
+  if (FUSE) {
+    if (tid < 64 && (int64_t)a.ap.pos >= j0 && (int64_t)a.ap.pos < j0 + n)
+      append_token<BKV_Q8_0, VF, RHAZ>(a.ap, a.ap.pos, 0, g, tid);
+  }
+  __syncthreads();
+  constexpr int RB = row_bytes(BKV_Q8_0);
+  u32x4 kr[4][4], ks[4];
+  int64_t ro[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    ro[i] = slot_of(L, j0 + min(64 * w + 16 * i + lr, n - 1)) * a.nkv + g;
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(L.kd + ro[i] * RB + 16 * lq);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) kr[i][j] = src[4 * j];
+    ks[i] = *reinterpret_cast<const u32x4 *>(L.ks + ro[i] * kScaleRowBytes);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  reinterpret_cast<float4 *>(s_q[w])[lane] = q4;
+  __builtin_amdgcn_wave_barrier();               // (wave h reads what it wrote: row h)
+  q8lim_build(&s_q[0][0], kHd, s_lim, s_lt, &s_wide, tid, NT);
+  lds_barrier();
+  float v[4], m = -INFINITY;
+  if (s_wide == 0u) {
+    // lane group lq holds dims 8 pq .. + 7 of each block once the halves have changed places
+    Q8Lim ql;
+    q8lim_load(s_lim, s_lt, ql, ((lq & 1) << 1) | (lq >> 1));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      long kb[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const auto x = __builtin_amdgcn_permlane32_swap(kr[i][j][0], kr[i][j][2], false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(kr[i][j][1], kr[i][j][3], false, false);
+        kb[2 * j] = (long)((unsigned long)x[0] | ((unsigned long)y[0] << 32));
+        kb[2 * j + 1] = (long)((unsigned long)x[1] | ((unsigned long)y[1] << 32));
+      }
+      v[i] = q8_score16r(kb, make_uint4(ks[i][0], ks[i][1], ks[i][2], ks[i][3]), ql.a, ql.t);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float r[kGqa];
+      q8_score_key_slow(reinterpret_cast<const uint32_t *>(L.kd + ro[i] * RB),
+                        reinterpret_cast<const uint32_t *>(L.ks + ro[i] * kScaleRowBytes), qg, a.qs, r);
+      v[i] = lq == 0 ? r[0] : lq == 1 ? r[1] : lq == 2 ? r[2] : r[3];
+    }
+  }
+  // scores of head lq, and the partition's (max, sum exp) used to place each key on the running sum
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int key = 64 * w + 16 * i + lr;
+    if (key < n) {
+      a.score[(size_t)(g * kGqa + lq) * a.ld + j0 + key] = v[i];
+      m = fmaxf(m, v[i] * a.scale);
+    }
+  }
+  m = row16_max(m);
+  if (lr == 0) s_max[w][lq] = m;
+  lds_barrier();
+  m = fmaxf(fmaxf(s_max[0][lq], s_max[1][lq]), fmaxf(s_max[2][lq], s_max[3][lq]));
+  float l = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (64 * w + 16 * i + lr < n) l += __expf(v[i] * a.scale - m);
+  l = row16_sum(l);
+  if (lr == 0) s_sum[w][lq] = l;
+  lds_barrier();
+  if (tid < kGqa)
+    a.stats[(size_t)(g * kGqa + tid) * a.nch + c] =
+        make_float2(fmaxf(fmaxf(s_max[0][tid], s_max[1][tid]), fmaxf(s_max[2][tid], s_max[3][tid])),
+                    (s_sum[0][tid] + s_sum[1][tid]) + (s_sum[2][tid] + s_sum[3][tid]));
+}
+
+// fp16 K: the tile in LDS, one serial chain per (key, head)
+template <int VF, bool FUSE, bool RHAZ>
+__global__ __launch_bounds__(kQkKeysF16) void qk_f16_kernel(QkArgs a) {
+  constexpr int NT = kQkKeysF16, DPR = 32, UPR = DPR + 1;   // data uint4 per K row, + pad (bank spread)
+  __shared__ uint4 tile[NT * UPR];
   __shared__ float red[NT / 64 + 1];
   const int c = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
-  const int64_t j0 = (int64_t)c * T::KEYS;
-  const int n = (int)min((int64_t)T::KEYS, (int64_t)a.nfill - j0);
+  const int64_t j0 = (int64_t)c * NT;
+  const int n = (int)min((int64_t)NT, (int64_t)a.nfill - j0);
   const LayerView &L = a.L;
 
   if (c == 0 && g == 0 && tid < a.nkv * kGqa) a.counters[tid * kCounterStride] = 0u;
   if (FUSE) {
     if (tid < 64 && (int64_t)a.ap.pos >= j0 && (int64_t)a.ap.pos < j0 + n)
-      append_token<KF, VF, RHAZ>(a.ap, a.ap.pos, 0, g, tid);
+      append_token<BKV_F16, VF, RHAZ>(a.ap, a.ap.pos, 0, g, tid);
     __syncthreads();
   }
-  constexpr int RB = row_bytes(KF);
-  stage_rows<NT, T::KEYS, T::DPR, T::UPR>(tile, L.kd, RB, L, a.nkv, g, j0, n);
-  if (KF == BKV_Q8_0) stage_rows<NT, T::KEYS, 1, T::UPR>(tile + 16, L.ks, kScaleRowBytes, L, a.nkv, g, j0, n);
+  constexpr int RB = row_bytes(BKV_F16);
+  stage_rows<NT, NT, DPR, UPR>(tile, L.kd, RB, L, a.nkv, g, j0, n);
   const float *qg = a.q + (size_t)g * kGqa * a.qs;
   float acc[kGqa];
-  if constexpr (KF == BKV_Q8_0) {
-    // the int8 matrix cores on the q rows' digits (bkv_q8dot.h)
-    __shared__ __attribute__((aligned(16))) int8_t s_lim[kLimBytes];
-    __shared__ int s_lt[kGqa];
-    __shared__ unsigned s_wide;
-    if (tid == 0) s_wide = 0u;
-    __syncthreads();
-    q8lim_build(qg, a.qs, s_lim, s_lt, &s_wide, tid, NT);
-    __syncthreads();                           // the digits and the K tile
-    if (s_wide == 0u) {
-      Q8Lim qlim;
-      q8lim_load(s_lim, s_lt, qlim);
-      q8_score64(tile + (tid & ~63) * T::UPR, T::UPR, qlim, acc);
-    } else {
-      q8_score_key_slow(tile + tid * T::UPR, qg, a.qs, acc);
-    }
-  } else {
+  {
     float qv[kGqa][kHd / 16];
     load_q16_rows(qg, qv, a.qs);
     __syncthreads();
     asm volatile("s_nop 4");      // DPP source registers written above: VALU-write -> DPP-read gap
-    qk_row_dot<KF>(tile + tid * T::UPR, qv, acc);
+    qk_row_dot<BKV_F16>(tile + tid * UPR, qv, acc);
   }
 
   // scores, and per head the partition's (max, sum exp) used to place each key on the running sum
@@ -113,13 +186,14 @@ __global__ __launch_bounds__(256) void e_kernel(EArgs a) {
   __shared__ int s_bin[kE2Chunk];
   __shared__ unsigned s_last;
   // walker staging (structure of arrays)
-  __shared__ long long w_ibase[kWalkBatch];
-  __shared__ int w_blast[kWalkBatch], w_cnt[kWalkBatch], w_off[kWalkBatch + 1];
-  __shared__ long long w_i[kWalkBatch * kMaxSpecial];
-  __shared__ long long w_k[kWalkBatch * kMaxSpecial];
-  __shared__ float w_e[kWalkBatch * kMaxSpecial];
-  __shared__ int w_b[kWalkBatch * kMaxSpecial];
-  __shared__ int w_du[kWalkBatch * kMaxSpecial];
+  __shared__ long long w_ibase[NT], w_tot;
+  __shared__ int w_blast[NT], w_cnt[NT], w_off[NT + 1];
+  __shared__ long long w_i[kWalkSpecials];
+  __shared__ long long w_k[kWalkSpecials];
+  __shared__ float w_e[kWalkSpecials];
+  __shared__ int w_b[kWalkSpecials];
+  __shared__ int w_du[kWalkSpecials];
+  static_assert(kWalkSpecials >= kMaxSpecial && kWalkSpecials >= NT, "a batch takes a chunk; the fallback's stage");
   const int c = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   const int64_t j0 = (int64_t)c * kE2Chunk;
   const int n = (int)min((int64_t)kE2Chunk, (int64_t)a.nfill - j0);
@@ -214,27 +288,35 @@ __global__ __launch_bounds__(256) void e_kernel(EArgs a) {
   long long i_prev = 0, k_prev = -1, ibase_run = 0;
   int blast_prev = kNoBinade;      // blast of the chunk before the current batch
   bool ok = true;
-  for (int cb = 0; cb < a.nch && ok; cb += kWalkBatch) {
-    const int nb = min(kWalkBatch, a.nch - cb);
+  for (int cb = 0, nb; cb < a.nch && ok; cb += nb) {
+    // a batch: the next chunks, one record per thread, as many as have kWalkSpecials specials together
+    // (nearly always all 256: a context of 262,144 keys in one batch)
+    const int nrec = min(NT, a.nch - cb);
     long long tot = 0;
     int cnt = 0;
-    if (tid < nb) {
+    if (tid < nrec) {
       const ChunkRec r = ld_rec(&a.rec[(size_t)h * a.nch + cb + tid]);
       tot = r.tot;
       cnt = r.nsp;
       w_blast[tid] = r.blast;
     }
-    long long tsum;
-    const long long ib = ibase_run + block_excl_scan<NT, long long>(tid < nb ? tot : 0, shl, &tsum);
-    int csum;
-    const int off = block_excl_scan<NT, int>(tid < nb ? min(cnt, kMaxSpecial) : 0, shi, &csum);
+    long long tall;
+    const long long ib = ibase_run + block_excl_scan<NT, long long>(tid < nrec ? tot : 0, shl, &tall);
+    int call;
+    const int off = block_excl_scan<NT, int>(tid < nrec ? min(cnt, kMaxSpecial) : 0, shi, &call);
+    nb = __syncthreads_count(tid < nrec && off + min(cnt, kMaxSpecial) <= kWalkSpecials);
     if (tid < nb) {
       w_ibase[tid] = ib;
       w_cnt[tid] = cnt;
       w_off[tid] = off;
+      if (tid == nb - 1) {
+        w_off[nb] = off + min(cnt, kMaxSpecial);
+        w_tot = ib + tot;
+      }
     }
-    if (tid == 0) w_off[nb] = csum;
     __syncthreads();
+    const int csum = w_off[nb];
+    const long long tnext = w_tot;
     TS(1);
     // one special per thread: its chunk by binary search over the offsets, then a single load
     for (int o = tid; o < csum; o += NT) {
@@ -312,7 +394,7 @@ __global__ __launch_bounds__(256) void e_kernel(EArgs a) {
     }
     TS(3);
     ok = s_last != 0;
-    ibase_run += tsum;
+    ibase_run = tnext;
     blast_prev = w_blast[nb - 1];
     __syncthreads();
   }
@@ -421,16 +503,22 @@ __global__ __launch_bounds__(256) void pv_kernel(PvArgs a) {
 
 // ------------------------------------------------------------------ partition merge + gate
 // gated = out * (1/(1 + exp(-gate))) (attn_vk.h:210-212)
+// One workgroup per head and 16 dims: 16 groups of threads each add every 16th partial (8 in flight), then
+// the groups are added in order. (64 workgroups of 4 groups, one load at a time, took 26 us for 391
+// partials, 4 now.)
 __global__ __launch_bounds__(256) void merge_kernel(RedArgs a) {
-  __shared__ float s[4][64];
+  __shared__ float s[16][17];
   const int h = blockIdx.x, tid = threadIdx.x;
-  const int d = blockIdx.y * 64 + (tid & 63), grp = tid >> 6;
+  const int d = blockIdx.y * 16 + (tid & 15), grp = tid >> 4;
   float acc = 0.0f;
-  for (int c = grp; c < a.nch; c += 4) acc += a.part[((size_t)c * a.nh + h) * kHd + d];
-  s[grp][tid & 63] = acc;
+#pragma unroll 8
+  for (int c = grp; c < a.nch; c += 16) acc += a.part[((size_t)c * a.nh + h) * kHd + d];
+  s[grp][tid & 15] = acc;
   __syncthreads();
-  if (tid < 64) {
-    const float v = (s[0][tid] + s[1][tid]) + (s[2][tid] + s[3][tid]);
+  if (tid < 16) {
+    float v = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v += s[i][tid];
     const size_t o = (size_t)h * kHd + d;
     a.out[o] = v;
     if (a.gate) a.out_gated[o] = v * (1.0f / (1.0f + exp_cr(-a.gate[gate_index(o, a.gs)])));
@@ -444,20 +532,22 @@ hipError_t launch_append(const AppendArgs &a, int kf, int vf, int n_tok, hipStre
   return hipGetLastError();
 }
 
-int qk_keys_per_wg(int kf) { return kf == BKV_Q8_0 ? QkTile<1>::KEYS : QkTile<0>::KEYS; }
+int qk_keys_per_wg(int kf) { return kf == BKV_Q8_0 ? kQkKeysQ8 : kQkKeysF16; }
 
 hipError_t launch_decode(const QkArgs &qa, const EArgs &ea, const PvArgs &pa, const RedArgs &ra,
                          int kf, int vf, bool fuse, hipStream_t st) {
   BKV_FMT_SWITCH(kf, vf, {
-    constexpr int NT = QkTile<KF_>::NT;
-    if (fuse)
-      hipLaunchKernelGGL((qk_kernel<KF_, VF_, true, false>), dim3(qa.nch, qa.nkv), dim3(NT), 0, st, qa);
-    else
-      hipLaunchKernelGGL((qk_kernel<KF_, VF_, false, false>), dim3(qa.nch, qa.nkv), dim3(NT), 0, st, qa);
+    if constexpr (KF_ == BKV_Q8_0) {
+      if (fuse) hipLaunchKernelGGL((qk_q8_kernel<VF_, true, false>), dim3(qa.nch, qa.nkv), dim3(kQkKeysQ8), 0, st, qa);
+      else hipLaunchKernelGGL((qk_q8_kernel<VF_, false, false>), dim3(qa.nch, qa.nkv), dim3(kQkKeysQ8), 0, st, qa);
+    } else {
+      if (fuse) hipLaunchKernelGGL((qk_f16_kernel<VF_, true, false>), dim3(qa.nch, qa.nkv), dim3(kQkKeysF16), 0, st, qa);
+      else hipLaunchKernelGGL((qk_f16_kernel<VF_, false, false>), dim3(qa.nch, qa.nkv), dim3(kQkKeysF16), 0, st, qa);
+    }
     hipLaunchKernelGGL(e_kernel, dim3(ea.nch, ea.nh), dim3(256), 0, st, ea);
     hipLaunchKernelGGL((pv_kernel<VF_>), dim3(pa.nch, pa.nkv), dim3(256), 0, st, pa);
   });
-  hipLaunchKernelGGL(merge_kernel, dim3(ra.nh, 4), dim3(256), 0, st, ra);
+  hipLaunchKernelGGL(merge_kernel, dim3(ra.nh, kHd / 16), dim3(256), 0, st, ra);
   return hipGetLastError();
 }
 

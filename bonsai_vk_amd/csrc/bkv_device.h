@@ -197,7 +197,9 @@ __device__ __forceinline__ void qk_row_dot(const uint4 *row, const float (&qv)[k
 // head walks the chunk records in order, adding increments exactly and specials in fp32, and checks
 // every binade assumption; if one fails it recomputes the serial loop itself.
 constexpr double kMargin = 1.0 / 16384.0;
-constexpr int kWalkBatch = 32;
+// specials the split path's walker holds at a time (its LDS sets how many workgroups a CU runs: 200,000 keys
+// in 63 us with 2048, 39 with 512; a row has a few dozen)
+constexpr int kWalkSpecials = 512;
 
 __device__ __forceinline__ void classify(double abefore, double aafter, float e, bool &special,
                                          int &bin, long long &inc) {

@@ -33,8 +33,7 @@ static inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 // 150.9-153.6, 64 154.0-156.0, 80 159.1-164.0; more than 128 leaves the short plan)
 constexpr int64_t kResMinKeysPerWg = 128;
 
-// Partition sizes of the split path. QK: the LDS K tile of one workgroup (256 q8_0 / 128 fp16
-// keys). Probability chunks: kE2Chunk keys. PV: enough workgroups to cover the chip (512 at nkv = 4)
+// Partition sizes of the split path. QK: the keys of one workgroup (256 q8_0 / 128 fp16). Probability chunks: kE2Chunk keys. PV: enough workgroups to cover the chip (512 at nkv = 4)
 // with 16..512 keys each. Every array is sized
 // by a bound that grows monotonically with n, so a workspace sized for max_ctx fits every n <= max_ctx.
 // BKV_DECODE forces a decode implementation where its plan fits: "split" (four launches),
@@ -61,7 +60,7 @@ static int prefill_splits(int nkv, int nqb, int64_t first_keys) {
 
 // BKV_PREFILL=mfma selects the matrix-core prefill (scores and sums in MFMA order: within
 // tolerance of the serial reference on long rows, not bit-identical probabilities); the default
-// is the exact path, one decode row per query.
+// is the exact path.
 static bool prefill_mfma_requested() {
   const char *e = std::getenv("BKV_PREFILL");
   return e && std::strcmp(e, "mfma") == 0;

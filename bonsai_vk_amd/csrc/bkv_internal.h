@@ -187,7 +187,7 @@ constexpr int kPxSlice = 512;    // queries per launch, at least (the score scra
 constexpr size_t kPxScratch = size_t(128) << 20;   // more queries per launch while their scores fit this
 constexpr int kPvQ = 32;         // queries per PV workgroup (4 kPvQ rows)
 constexpr int kPvSplit = 4;      // PV key ranges a slice of kPxSlice queries may have (shorter: more)
-constexpr int kPxMinQ = 16;      // shorter chunks run as decode rows
+constexpr int kPxMinQ = 16;      // shorter chunks run as decode rows where those take less (px_worthwhile)
 
 struct PrefillXArgs {
   LayerView L;

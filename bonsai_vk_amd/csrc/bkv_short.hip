@@ -463,7 +463,9 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
     // has read that one; later tiles are waited for in order, the younger ones' loads left in flight.
     if (t == 0) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (VF && append && w == (kend - 1) >> 6 && lane == 0) s_vs[kend - 1] = s_row[1][16];
+      // (the appended token's scales, also for the padding after it: those entries were loaded from its slot,
+      // which may have held anything, and p = 0 times a NaN scale is NaN)
+      if (VF && append && w == (kend - 1) >> 6 && lane >= ((kend - 1) & 63)) s_vs[64 * w + lane] = s_row[1][16];
       lds_barrier();                               // every wave's rows, and p16
     } else if (nt > NB) {
       if (t >= NB) {
@@ -475,14 +477,18 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
     }
     char *vt = s_v[t % NB];
     if (append && t == nt - 1) {                   // the appended row, this wave's dims, over its loaded copy
-      const int r = (kend - 1) & 63, i = r >> 2;
+      const int r = (kend - 1) & 63;
       if constexpr (VF) {
+        const int i = r >> 2;
         if (lane < 2)
           *reinterpret_cast<uint4 *>(vt + 1024 * i + 64 * ((2 * w + lane) ^ (i & 3)) + 16 * (r & 3)) = s_row[1][2 * w + lane];
-      } else {
-        if (lane < 4)
-          *reinterpret_cast<uint4 *>(vt + 1024 * (i + 16 * (w >> 2)) + 64 * ((4 * (w & 3) + lane) ^ (2 * ((i >> 1) & 3))) +
-                                     16 * (r & 3)) = s_row[1][4 * w + lane];
+      } else {                                     // (and over the padding's copies: see the scales)
+        const int c = 4 * (w & 3) + (lane & 3);
+        for (int rr = r + (lane >> 2); rr < 64; rr += 16) {
+          const int i = rr >> 2;
+          *reinterpret_cast<uint4 *>(vt + 1024 * (i + 16 * (w >> 2)) + 64 * (c ^ (2 * ((i >> 1) & 3))) + 16 * (rr & 3)) =
+              s_row[1][4 * w + (lane & 3)];
+        }
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }

@@ -98,3 +98,24 @@ def test_short_prefill(kf, vf, pos0, n, page, kind, monkeypatch):
         torch.cuda.synchronize()
         assert float((out[i] - want).abs().max()) <= tol, i
         assert float((og[i] - wg).abs().max()) <= tol, i
+
+
+# a first token, a token in the middle of a tile, the last of a tile, the first of a tile
+@pytest.mark.parametrize("kf,vf", FMTS)
+@pytest.mark.parametrize("n", [1, 2, 40, 64, 65, 300])
+def test_short_decode_step_into_unwritten_slots(kf, vf, n):
+    """What the appended token's slot and those after it held before (here NaN bytes) reaches no output."""
+    say(f"short decode into NaN slots kf={kf} vf={vf} n={n}")
+    outs = []
+    k, v = (torch.from_numpy(x).cuda() for x in oracle.synth_kv(n, 4, 256, 3, 0, outliers=3))
+    q = queries(1, "normal")[0]
+    for fill in (0, 255):
+        c = KvCache(n_layers=1, cap=n + 70, k_fmt=kf, v_fmt=vf, max_ctx=n + 70)
+        for t in (c.k_data, c.k_scales, c.v_data, c.v_scales):
+            if t is not None:
+                t.fill_(fill)
+        if n > 1:
+            c.append(0, 0, k[:n - 1], v[:n - 1])
+        outs.append(c.decode_step(0, n - 1, k[n - 1:], v[n - 1:], q)[0])
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(outs[0]).all()) and torch.equal(outs[0], outs[1])

@@ -52,6 +52,57 @@ __device__ __forceinline__ void split_prod(h2 b, h2 s, h2 &hi, h2 &lo) {
   lo = __builtin_elementwise_fma(b, s, -hi);
 }
 
+// ---------------------------------------------------------------- q8_0 V tiles outside the plain products
+// The PV kernels multiply p16 with d * b split into two fp16 operands. A scale of 512 or more (scale_big)
+// takes the products out of fp16's range; a tile that holds one goes through pv_tile_careful, where such a
+// key enters a second pair of operands as (d * 2^-8) * b against p16 * 2^8, both exact (d is at least 2
+// there, p16 at most 1). It costs twice the MFMAs; ordinary values never have such a tile. (us, without and
+// with the test for it, and with every scale past 512: a decode of 300 keys 12.9 / 12.9 / 17.0, of 447
+// 17.4 / 17.5 / 23.0, 512 queries onto 8192 keys 334 / 335 / 430.)
+
+// bits 14 and 30: the low and high fp16 of w is 512 or more in magnitude, Inf or NaN
+__device__ __forceinline__ uint32_t scale_big(uint32_t w) { return w & (w << 1) & 0x40004000u; }
+// bits 15 and 31: the low and high fp16 of w is Inf or NaN
+__device__ __forceinline__ uint32_t non_finite(uint32_t w) { return ((w & 0x7C007C00u) + 0x04000400u) & 0x80008000u; }
+// 0xFFFF in the halves whose flag (bit N of each) is set
+template <int N>
+__device__ __forceinline__ uint32_t half_mask(uint32_t flags) { return (flags >> N) * 0xFFFFu; }
+
+// One 64-key tile against NTR tiles of 16 rows: lane l's accumulators o[mt][nt] hold row 16 nt + l % 16.
+// ops(ks, mt, x, s): the bytes x and scales s, as fp16, of the lane's keys 32 ks + 8 (l / 16) .. + 7 in pairs;
+// rows(ks, nt): their p16.
+template <int NTR, typename OPS, typename ROWS>
+__device__ __forceinline__ void pv_tile_careful(f4 (&o)[2][NTR], const OPS &ops, const ROWS &rows) {
+#pragma unroll 1
+  for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      uint32_t x[4], s[4], a[4][4];
+      ops(ks, mt, x, s);
+#pragma unroll
+      for (int pp = 0; pp < 4; ++pp) {
+        const uint32_t big = half_mask<14>(scale_big(s[pp]));
+        h2 hi, lo;
+        split_prod(as_h2(x[pp]), as_h2(s[pp] & ~big), hi, lo);
+        a[0][pp] = as_u(hi);
+        a[1][pp] = as_u(lo);
+        split_prod(as_h2(x[pp]), as_h2(s[pp] & big) * h2{(_Float16)0x1p-8f, (_Float16)0x1p-8f}, hi, lo);
+        a[2][pp] = as_u(hi);
+        a[3][pp] = as_u(lo) & ~half_mask<15>(non_finite(as_u(hi)));     // (Inf - Inf: the Inf is in hi)
+      }
+#pragma unroll
+      for (int nt = 0; nt < NTR; ++nt) {
+        const h8 p = rows(ks, nt);
+        const _Float16 f = (_Float16)256.0f;
+        const h8 pb = p * h8{f, f, f, f, f, f, f, f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          o[mt][nt] = mfma16(__builtin_bit_cast(h8, make_uint4(a[i][0], a[i][1], a[i][2], a[i][3])), i < 2 ? p : pb, o[mt][nt]);
+      }
+    }
+  }
+}
+
 // Workgroup barrier for LDS traffic only: every wave's LDS operations have completed, while its
 // global loads (prefetches a step or more ahead) stay in flight. __syncthreads() also releases
 // global memory, i.e. waits for every outstanding load and store of the wave first, which would

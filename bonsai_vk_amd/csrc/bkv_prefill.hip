@@ -1056,8 +1056,8 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
                    : "memory", "m0");
     }
   };
-  auto tile = [&](int t, const PvIn &in) {
-    char *pb = s_p + (t & 1) * (R * kPfRS);
+  // tile t's p16 into the P buffer pb, its block scales into vsk
+  auto probs = [&](const PvIn &in, char *pb, uint32_t (&vsk)[16]) {
     float ev[RPW];
 #pragma unroll
     for (int i = 0; i < RPW / 4; ++i) {
@@ -1069,12 +1069,52 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
       *reinterpret_cast<_Float16 *>(pb + (RPW * w + i) * kPfRS + 2 * pk) = h;
     }
     // the block scales of the lane's 16 keys: key (ks, c) from lane 8 ks + c of its row
-    uint32_t vsk[16];
     if constexpr (VF) {
 #define BKV_BC(i) vsk[i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)in.vs, 0x150 + (i), 0xF, 0xF, false)
       BKV_BC(0); BKV_BC(1); BKV_BC(2); BKV_BC(3); BKV_BC(4); BKV_BC(5); BKV_BC(6); BKV_BC(7);
       BKV_BC(8); BKV_BC(9); BKV_BC(10); BKV_BC(11); BKV_BC(12); BKV_BC(13); BKV_BC(14); BKV_BC(15);
 #undef BKV_BC
+    }
+  };
+  // tile t's V values of key half ks and dim tile mt as LDS holds them, and from them the operand in pairs of
+  // keys (see pv_tile_careful): pair p holds keys 2p, 2p+1 of the lane's 8
+  auto vread = [&](int t, int ks, int mt) {
+    const uint32_t vb = vbase + (uint32_t)VB * (uint32_t)(t % 3) + (ks ? vrd[1] : vrd[0]);
+    if constexpr (VF) {
+      const v2i_t bv = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+          (__attribute__((address_space(3))) v2i_t *)(uintptr_t)(vb ^ (uint32_t)(64 * (2 * w + mt))));
+      return make_uint4((uint32_t)bv.x, (uint32_t)bv.y, 0u, 0u);
+    } else {
+      // keys 8 lq .. + 3 of the half from one block, + 4 .. + 7 from the next (the same swizzle)
+      const uint32_t ad = vb ^ (uint32_t)(128 * (2 * (w & 3) + mt));
+      const v4s_t r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)ad);
+      const v4s_t r1 =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)(ad + 1024u));
+      return __builtin_bit_cast(uint4, (v8s_t){r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]});
+    }
+  };
+  auto operand = [&](const uint4 &v, int ks, const uint32_t (&vsk)[16], uint32_t (&x)[4], uint32_t (&s)[4]) {
+    if constexpr (VF) {
+      constexpr uint32_t kSel[4] = {0x0C010C00u, 0x0C030C02u, 0x0C050C04u, 0x0C070C06u};
+#pragma unroll
+      for (int pp = 0; pp < 4; ++pp) {
+        const uint32_t bw = __builtin_amdgcn_perm(v.y, v.x, kSel[pp]) ^ 0x64806480u;
+        x[pp] = as_u(as_h2(bw) - h2{(_Float16)1152.0f, (_Float16)1152.0f});
+        s[pp] = ks ? vsk[8 + 2 * pp] | (vsk[9 + 2 * pp] << 16) : vsk[2 * pp] | (vsk[1 + 2 * pp] << 16);
+      }
+    } else {
+      x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+    }
+  };
+  __shared__ __attribute__((aligned(8))) uint8_t s_careful[2][8];   // [t % 2][wave]: tile t needs pv_tile_careful
+  // true: the tile was left out, as it needs pv_tile_careful
+  auto tile = [&](int t, const PvIn &in) {
+    char *pb = s_p + (t & 1) * (R * kPfRS);
+    uint32_t vsk[16];
+    probs(in, pb, vsk);
+    if constexpr (VF) {
+      const bool big = __any(scale_big(in.vs) != 0u);
+      if (lane == 0) s_careful[t & 1][w] = big;
     }
     // this wave's V rows of tile t have landed when at most the loads issued after them are in
     // flight: tile t + 1's register loads (NL) and rows (ND), tile t + 2's register loads (NL)
@@ -1083,36 +1123,33 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
     asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
     lds_barrier();                                  // the P tile and every wave's V rows of tile t
     dma_tile(t + 2);                                // (its buffer's last readers, tile t - 1, are done)
-    const uint32_t vb = vbase + (uint32_t)VB * (uint32_t)(t % 3);
-    // the A operands (registers only): pair p of key half ks holds keys 2p, 2p+1
+    unsigned long careful = 0;
+    if (VF) careful = *reinterpret_cast<const unsigned long *>(s_careful[t & 1]);
+    uint4 v[2][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i >> 1][i & 1] = vread(t, i >> 1, i & 1);
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane((int)(careful | (careful >> 32))) != 0, 0)) return true;
+    // the A operands (registers only)
     h8 ah[2][2], al[2][2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
+        uint32_t x[4], s[4];
+        operand(v[ks][mt], ks, vsk, x, s);
         if constexpr (VF) {
-          const v2i_t bv = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-              (__attribute__((address_space(3))) v2i_t *)(uintptr_t)((vb + vrd[ks]) ^ (uint32_t)(64 * (2 * w + mt))));
-          constexpr uint32_t kSel[4] = {0x0C010C00u, 0x0C030C02u, 0x0C050C04u, 0x0C070C06u};
           uint32_t hw[4], lw[4];
 #pragma unroll
           for (int pp = 0; pp < 4; ++pp) {
-            const uint32_t bw = __builtin_amdgcn_perm((uint32_t)bv.y, (uint32_t)bv.x, kSel[pp]) ^ 0x64806480u;
-            const h2 x = as_h2(bw) - h2{(_Float16)1152.0f, (_Float16)1152.0f};
             h2 hi, lo;
-            split_prod(x, as_h2(vsk[8 * ks + 2 * pp] | (vsk[8 * ks + 2 * pp + 1] << 16)), hi, lo);
+            split_prod(as_h2(x[pp]), as_h2(s[pp]), hi, lo);
             hw[pp] = as_u(hi);
             lw[pp] = as_u(lo);
           }
           ah[ks][mt] = __builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3]));
           al[ks][mt] = __builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3]));
         } else {
-          // keys 8 lq .. + 3 of the half from one block, + 4 .. + 7 from the next (the same swizzle)
-          const uint32_t ad = (vb + vrd[ks]) ^ (uint32_t)(128 * (2 * (w & 3) + mt));
-          const v4s_t r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)ad);
-          const v4s_t r1 =
-              __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)(ad + 1024u));
-          ah[ks][mt] = __builtin_bit_cast(h8, (v8s_t){r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]});
+          ah[ks][mt] = __builtin_bit_cast(h8, make_uint4(x[0], x[1], x[2], x[3]));
         }
       }
     }
@@ -1128,12 +1165,14 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
         }
       }
     }
+    return false;
   };
   // three register sets and V buffers, each tile's operands requested two tiles ahead (branch-free
   // groups of three, so that the compiler's wait counting keeps the two younger tiles' loads in
   // flight); the V rows of tile t + 2 go out once every wave has passed tile t's barrier
   if (t0 < t1) {
     PvIn in[3];
+    int tc = t1;                                    // the first tile that needs pv_tile_careful
     load_tile(t0, in[0]);
     dma_tile(t0);
     load_tile(t0 + 1, in[1]);
@@ -1143,10 +1182,29 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
       for (int u = 0; u < 3; ++u) {
         load_tile(t + u + 2, in[(u + 2) % 3]);
         __builtin_amdgcn_sched_barrier(0);
-        tile(t + u, in[u]);
+        if (tile(t + u, in[u])) {                   // (the same in every wave)
+          tc = t + u;
+          t = t1;
+          break;
+        }
       }
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last rows landed before the LDS is released
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last rows landed before the LDS is used again or released
+    // from that tile on one after the other
+#pragma unroll 1
+    for (int t = tc; t < t1; ++t) {
+      lds_barrier();                                // the buffers' last readers are done
+      uint32_t vsk[16];
+      load_tile(t, in[0]);
+      dma_tile(t);
+      probs(in[0], s_p, vsk);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();
+      pv_tile_careful<NTR>(
+          o,
+          [&](int ks, int mt, uint32_t (&x)[4], uint32_t (&s)[4]) { operand(vread(t, ks, mt), ks, vsk, x, s); },
+          [&](int ks, int nt) { return *reinterpret_cast<const h8 *>(s_p + (16 * nt + lr) * kPfRS + 2 * (32 * ks + 8 * lq)); });
+    }
   }
   // lane l holds out^T[dim 32 w + 16 mt + 4(l/16) + r][row 16 nt + l%16] in o[mt][nt][r]: the range's
   // partial, or (one range) the output

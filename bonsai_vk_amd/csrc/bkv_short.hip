@@ -54,6 +54,7 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
   __shared__ float s_ex[16], s_red[8][NR], s_sum[NR];
   __shared__ int s_lt[kGqa];
   __shared__ unsigned s_flags, s_wide;
+  __shared__ __attribute__((aligned(8))) uint8_t s_big[8];   // (q8_0 V) tile t has a scale past the plain products
   if (tid == 0) { s_flags = 0u; s_wide = 0u; }
   if (tid < 32) s_t2[tid] = kExp2Tab[tid];
   static_assert(16 * kShPS >= kQ8fUnit * 16 && 16 * kShPS >= kHd * 16 * 4 && 16 * kShPS >= kLimBytes, "q16 operands in s_p");
@@ -457,7 +458,8 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
                            8 * (lane & 1));
     }
   }
-  f4 o[2] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+  f4 o[2][1] = {{f4{0.f, 0.f, 0.f, 0.f}}, {f4{0.f, 0.f, 0.f, 0.f}}};
+  unsigned long big = 0;                           // byte t: s_big
   for (int t = 0; t < nt; ++t) {
     // The first NB tiles have landed at t = 0. Tile t + NB - 1 goes into tile t - 1's buffer once every wave
     // has read that one; later tiles are waited for in order, the younger ones' loads left in flight.
@@ -466,7 +468,13 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
       // (the appended token's scales, also for the padding after it: those entries were loaded from its slot,
       // which may have held anything, and p = 0 times a NaN scale is NaN)
       if (VF && append && w == (kend - 1) >> 6 && lane >= ((kend - 1) & 63)) s_vs[64 * w + lane] = s_row[1][16];
+      if (VF && w < nt) {
+        const uint4 s = s_vs[64 * w + lane];
+        const bool b = __any((scale_big(s.x) | scale_big(s.y) | scale_big(s.z) | scale_big(s.w)) != 0u);
+        if (lane == 0) s_big[w] = b;
+      }
       lds_barrier();                               // every wave's rows, and p16
+      if (VF) big = *reinterpret_cast<const unsigned long *>(s_big);
     } else if (nt > NB) {
       if (t >= NB) {
         if (t + 1 >= nt) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -493,50 +501,68 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     const uint32_t vb = vbase + (uint32_t)VB * (uint32_t)(t % NB);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const h8 bp = *reinterpret_cast<const h8 *>(s_p + lr * kShPS + 2 * (64 * t + 32 * ks + 8 * lq));
-      uint32_t vsk[8];
+    auto rows = [&](int ks, int) { return *reinterpret_cast<const h8 *>(s_p + lr * kShPS + 2 * (64 * t + 32 * ks + 8 * lq)); };
+    // the V operand in pairs of keys (see pv_tile_careful)
+    auto ops = [&](int ks, int mt, uint32_t (&x)[4], uint32_t (&s)[4]) {
       if constexpr (VF) {
+        const uint16_t *vs = reinterpret_cast<const uint16_t *>(&s_vs[64 * t + 32 * ks + 8 * lq]) + w;
+        const v2i_t bv = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+            (__attribute__((address_space(3))) v2i_t *)(uintptr_t)((vb + vrd[ks]) ^ (uint32_t)(64 * (2 * w + mt))));
+        constexpr uint32_t kSel[4] = {0x0C010C00u, 0x0C030C02u, 0x0C050C04u, 0x0C070C06u};
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
-          vsk[c] = reinterpret_cast<const uint16_t *>(&s_vs[64 * t + 32 * ks + 8 * lq + c])[w];
+        for (int pp = 0; pp < 4; ++pp) {
+          const uint32_t bw = __builtin_amdgcn_perm((uint32_t)bv.y, (uint32_t)bv.x, kSel[pp]) ^ 0x64806480u;
+          x[pp] = as_u(as_h2(bw) - h2{(_Float16)1152.0f, (_Float16)1152.0f});
+          s[pp] = (uint32_t)vs[16 * pp] | ((uint32_t)vs[16 * pp + 8] << 16);
+        }
+      } else {
+        const uint32_t ad = (vb + vrd[ks]) ^ (uint32_t)(128 * (2 * (w & 3) + mt));
+        const v4s_t r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)ad);
+        const v4s_t r1 =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)(ad + 1024u));
+        const uint4 v = __builtin_bit_cast(uint4, (v8s_t){r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]});
+        x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
       }
+    };
+    uint32_t x[2][2][4], s[2][4];
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        if constexpr (VF) {
-          const v2i_t bv = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-              (__attribute__((address_space(3))) v2i_t *)(uintptr_t)((vb + vrd[ks]) ^ (uint32_t)(64 * (2 * w + mt))));
-          constexpr uint32_t kSel[4] = {0x0C010C00u, 0x0C030C02u, 0x0C050C04u, 0x0C070C06u};
-          uint32_t hw[4], lw[4];
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-          for (int pp = 0; pp < 4; ++pp) {
-            const uint32_t bw = __builtin_amdgcn_perm((uint32_t)bv.y, (uint32_t)bv.x, kSel[pp]) ^ 0x64806480u;
-            const h2 x = as_h2(bw) - h2{(_Float16)1152.0f, (_Float16)1152.0f};
-            h2 hi, lo;
-            split_prod(x, as_h2(vsk[2 * pp] | (vsk[2 * pp + 1] << 16)), hi, lo);
-            hw[pp] = as_u(hi);
-            lw[pp] = as_u(lo);
+      for (int mt = 0; mt < 2; ++mt) ops(ks, mt, x[ks][mt], s[ks]);
+    if (VF && (__builtin_amdgcn_readfirstlane((int)(big >> (8 * t))) & 0xFF) != 0) {
+      pv_tile_careful<1>(o, ops, rows);
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const h8 bp = rows(ks, 0);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          const uint32_t (&xk)[4] = x[ks][mt];
+          if constexpr (VF) {
+            uint32_t hw[4], lw[4];
+#pragma unroll
+            for (int pp = 0; pp < 4; ++pp) {
+              h2 hi, lo;
+              split_prod(as_h2(xk[pp]), as_h2(s[ks][pp]), hi, lo);
+              hw[pp] = as_u(hi);
+              lw[pp] = as_u(lo);
+            }
+            o[mt][0] = mfma16(__builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3])), bp, o[mt][0]);
+            o[mt][0] = mfma16(__builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3])), bp, o[mt][0]);
+          } else {
+            o[mt][0] = mfma16(__builtin_bit_cast(h8, make_uint4(xk[0], xk[1], xk[2], xk[3])), bp, o[mt][0]);
           }
-          o[mt] = mfma16(__builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3])), bp, o[mt]);
-          o[mt] = mfma16(__builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3])), bp, o[mt]);
-        } else {
-          const uint32_t ad = (vb + vrd[ks]) ^ (uint32_t)(128 * (2 * (w & 3) + mt));
-          const v4s_t r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)ad);
-          const v4s_t r1 =
-              __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)(ad + 1024u));
-          o[mt] = mfma16(__builtin_bit_cast(h8, (v8s_t){r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]}), bp, o[mt]);
         }
       }
     }
   }
-  // lane l holds out^T[dim 32 w + 16 mt + 4 lq + i][row lr] in o[mt][i]
+  // lane l holds out^T[dim 32 w + 16 mt + 4 lq + i][row lr] in o[mt][0][i]
   if (lr < NR && (lr >> 2) < nqv) {
     const size_t row = (size_t)(q0 + (lr >> 2)) * a.nh + g * kGqa + (lr & 3);
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
       const int d = 32 * w + 16 * mt + 4 * lq;
-      const float4 v = make_float4(o[mt][0], o[mt][1], o[mt][2], o[mt][3]);
+      const float4 v = make_float4(o[mt][0][0], o[mt][0][1], o[mt][0][2], o[mt][0][3]);
       *reinterpret_cast<float4 *>(a.out + row * kHd + d) = v;
       if (a.gate) {
         float4 f;

@@ -1106,6 +1106,7 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
       x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
     }
   };
+  const int lim0 = (int)(a.pos0 + (uint32_t)q0);   // the first query's last key
   __shared__ __attribute__((aligned(8))) uint8_t s_careful[2][8];   // [t % 2][wave]: tile t needs pv_tile_careful
   // true: the tile was left out, as it needs pv_tile_careful
   auto tile = [&](int t, const PvIn &in) {
@@ -1121,10 +1122,22 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
     constexpr int NL = RPW / 4 + (VF ? 1 : 0);
     static_assert(2 * NL + ND == 12, "the wait count below");
     asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    // some rows do not see some of the tile's keys, or it is past the range (t1 - 1 again, with p = 0)
+    const bool masked = kPfTile * t + kPfTile - 1 > lim0 || t >= t1;
+    if (!VF && masked) {                            // the values this wave loaded
+      uint32_t nf = 0;
+#pragma unroll
+      for (int u = 0; u < ND; ++u) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(s_v[t % 3] + 1024 * (2 * w + (u & 1) + 16 * (u >> 1)) + 16 * lane);
+        nf |= non_finite(v.x) | non_finite(v.y) | non_finite(v.z) | non_finite(v.w);
+      }
+      const bool bad = __any(nf != 0u);
+      if (lane == 0) s_careful[t & 1][w] = bad;
+    }
     lds_barrier();                                  // the P tile and every wave's V rows of tile t
     dma_tile(t + 2);                                // (its buffer's last readers, tile t - 1, are done)
     unsigned long careful = 0;
-    if (VF) careful = *reinterpret_cast<const unsigned long *>(s_careful[t & 1]);
+    if (VF || masked) careful = *reinterpret_cast<const unsigned long *>(s_careful[t & 1]);
     uint4 v[2][2];
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i >> 1][i & 1] = vread(t, i >> 1, i & 1);
@@ -1200,8 +1213,8 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
       probs(in[0], s_p, vsk);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       lds_barrier();
-      pv_tile_careful<NTR>(
-          o,
+      pv_tile_careful<VF, NTR, kPxQ>(
+          o, kPfTile * t, lim0, kPfTile * t + kPfTile - 1 > lim0,
           [&](int ks, int mt, uint32_t (&x)[4], uint32_t (&s)[4]) { operand(vread(t, ks, mt), ks, vsk, x, s); },
           [&](int ks, int nt) { return *reinterpret_cast<const h8 *>(s_p + (16 * nt + lr) * kPfRS + 2 * (32 * ks + 8 * lq)); });
     }

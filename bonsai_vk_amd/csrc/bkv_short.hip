@@ -501,6 +501,8 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     const uint32_t vb = vbase + (uint32_t)VB * (uint32_t)(t % NB);
+    const int lim0 = (int)a.pos0 + q0;             // the first query's last key
+    const bool masked = 64 * t + 63 > lim0;        // some rows do not see some of the tile's keys
     auto rows = [&](int ks, int) { return *reinterpret_cast<const h8 *>(s_p + lr * kShPS + 2 * (64 * t + 32 * ks + 8 * lq)); };
     // the V operand in pairs of keys (see pv_tile_careful)
     auto ops = [&](int ks, int mt, uint32_t (&x)[4], uint32_t (&s)[4]) {
@@ -529,8 +531,17 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) ops(ks, mt, x[ks][mt], s[ks]);
-    if (VF && (__builtin_amdgcn_readfirstlane((int)(big >> (8 * t))) & 0xFF) != 0) {
-      pv_tile_careful<1>(o, ops, rows);
+    bool careful = false;
+    if constexpr (VF) {
+      careful = (__builtin_amdgcn_readfirstlane((int)(big >> (8 * t))) & 0xFF) != 0;
+    } else if (masked) {
+      uint32_t nf = 0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) nf |= non_finite(x[i >> 3][(i >> 2) & 1][i & 3]);
+      careful = __any(nf != 0u);
+    }
+    if (careful) {
+      pv_tile_careful<VF, 1, NQ>(o, 64 * t, lim0, masked, ops, rows);
     } else {
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {

@@ -1,6 +1,7 @@
-"""GPU: V past the range of fp16 products in short decodes and chunks against the oracle.
+"""GPU: V past the range of fp16 products, and non-finite V, in short decodes and chunks against the oracle.
 
-A q8_0 block holds scale * byte up to 8.3 million while fp16 ends at 65504. Bar: 1e-4 of the block's largest output, block by block
+A q8_0 block holds scale * byte up to 8.3 million while fp16 ends at 65504, and a chunk's rows share the
+tiles of keys that only some of them see. Bar: 1e-4 of the block's largest output, block by block
 (every 32 dimensions have a scale of their own, so a large block must not cover for a small one)."""
 import numpy as np
 import pytest
@@ -63,3 +64,38 @@ def test_q8v_past_fp16(pos0, n, kind, kf):
     r = oracle.rel_err(out.reshape(-1, 32), want.reshape(-1, 32))
     say(f"  max err of a block's largest {r:.2e}")
     assert r <= TOL
+
+
+@pytest.mark.parametrize("kf,vf", [(BKV_Q8_0, BKV_Q8_0), (BKV_F16, BKV_F16)])
+@pytest.mark.parametrize("what", [np.inf, np.nan, -1e9])
+@pytest.mark.parametrize("pos0,n", [s for s in SHAPES if s[1] > 1] + [(100, 40)])
+def test_later_tokens_non_finite_v(pos0, n, what, kf, vf):
+    """A token whose V is stored as Inf or NaN (also a value past the format's range) in the last token of a
+    chunk and in one before it: the queries before each are what they are without it, bit for bit, and the
+    others are finite, Inf and NaN where the oracle is."""
+    say(f"non-finite V: pos0={pos0} n={n} {what} kf={kf} vf={vf}")
+    m = pos0 + n
+    v = oracle.synth_kv(m, 4, 256, 9, 0, outliers=3)[1]
+    first = m - 1 - min(n - 1, 2) // 2                 # (the chunk's last token, or the one before it too)
+    bad = v.copy()
+    bad[m - 1, :, 40:72] = what
+    bad[first, 1, 7] = what
+    plain, _ = both(*filled(pos0, n, kf, vf, v), pos0, n)
+    dev, host = filled(pos0, n, kf, vf, bad)
+    out, want = both(dev, host, pos0, n)
+    assert np.array_equal(out[:first - pos0], plain[:first - pos0])
+    assert np.array_equal(np.isnan(out), np.isnan(want)) and np.array_equal(np.isinf(out), np.isinf(want))
+    ok = np.isfinite(want)
+    assert np.array_equal(np.sign(out[np.isinf(want)]), np.sign(want[np.isinf(want)]))
+    assert np.abs(out[ok] - want[ok]).max() <= TOL * np.abs(want[ok]).max()
+
+
+@pytest.mark.parametrize("kf,vf", [(BKV_Q8_0, BKV_Q8_0), (BKV_F16, BKV_F16)])
+@pytest.mark.parametrize("nfill", [1, 40, 64, 300])
+def test_short_decode_of_a_non_finite_last_key(nfill, kf, vf):
+    """The key a decode's padding repeats holds Inf: the output is Inf where the oracle's is, not NaN."""
+    say(f"non-finite last key nfill={nfill} kf={kf} vf={vf}")
+    v = oracle.synth_kv(nfill, 4, 256, 9, 0, outliers=3)[1]
+    v[nfill - 1, :, 3] = -1e9 if vf == BKV_Q8_0 else np.inf
+    out, want = both(*filled(nfill - 1, 1, kf, vf, v), nfill - 1, 1)
+    assert np.array_equal(np.isnan(out), np.isnan(want)) and np.array_equal(np.isinf(out), np.isinf(want))

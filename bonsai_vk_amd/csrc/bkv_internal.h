@@ -185,7 +185,7 @@ constexpr int kPxTile = 64;      // keys per score tile, q8_0 K
 constexpr int kPxTile16 = 256;   // keys per score tile, fp16 K (and the scratch's granularity)
 constexpr int kPxSlice = 512;    // queries per launch, at least (the score scratch holds them)
 constexpr size_t kPxScratch = size_t(128) << 20;   // more queries per launch while their scores fit this
-constexpr int kPvQ = 32;         // queries per PV workgroup (4 kPvQ rows)
+constexpr int kPvQ = 32;         // queries per PV workgroup (4 kPvQ rows; half of it in slices of at most that)
 constexpr int kPvSplit = 4;      // PV key ranges a slice of kPxSlice queries may have (shorter: more)
 constexpr int kPxMinQ = 16;      // shorter chunks run as decode rows where those take less (px_worthwhile)
 

@@ -60,9 +60,9 @@ __device__ __forceinline__ void split_prod(h2 b, h2 s, h2 &hi, h2 &lo) {
 //  * keys that some of the rows do not see (later queries' keys, padding) beside a value that is Inf or
 //    NaN: p = 0 does not take them out, as 0 * Inf is NaN. The rows of one query at a time are computed with
 //    the keys past that query's last one zeroed in the V operand, and the other rows' results dropped.
-// A tile of either kind costs up to 2 x 4 times the MFMAs; ordinary values never have one. (us, without and
-// with the test for large scales, and with every scale past 512: a decode of 300 keys 12.9 / 12.9 / 17.0, of
-// 447 17.4 / 17.5 / 23.0, 512 queries onto 8192 keys 334 / 335 / 430.)
+// A tile of either kind costs up to 2 x 4 times the MFMAs; ordinary values never have one. (us, with ordinary
+// scales and with every scale past 512: a decode of 300 keys 13.2 / 19.1, 6 queries onto 300 keys 16.8 / 26.5,
+// 6 onto 3000 47.2 / 59.0, 512 onto 8192 333 / 430.)
 
 // bits 14 and 30: the low and high fp16 of w is 512 or more in magnitude, Inf or NaN
 __device__ __forceinline__ uint32_t scale_big(uint32_t w) { return w & (w << 1) & 0x40004000u; }
@@ -74,12 +74,13 @@ __device__ __forceinline__ uint32_t half_mask(uint32_t flags) { return (flags >>
 
 // One 64-key tile (first key key0) against NTR tiles of 16 rows: lane l's accumulators o[mt][nt] hold row
 // 16 nt + l % 16, i.e. the chunk's query 4 nt + (l % 16) / 4, whose last key is lim0 + 4 nt + (l % 16) / 4.
+// l: the accumulators of the products' small parts (o itself will do).
 // masked: some row does not see all of the tile's keys (NQ queries per row tile). ops(ks, mt, x, s): the V
 // operand of the lane's keys key0 + 32 ks + 8 (l / 16) .. + 7 in pairs: fp16 V x; q8_0 V the bytes x and
 // scales s as fp16. rows(ks, nt): their p16.
 template <int VF, int NTR, int NQ, typename OPS, typename ROWS>
-__device__ __forceinline__ void pv_tile_careful(f4 (&o)[2][NTR], int key0, int lim0, bool masked, const OPS &ops, const ROWS &rows) {
-  constexpr int NA = VF ? 4 : 1;
+__device__ __forceinline__ void pv_tile_careful(f4 (&o)[2][NTR], f4 (&l)[2][NTR], int key0, int lim0, bool masked, const OPS &ops, const ROWS &rows) {
+  constexpr int NA = VF ? 4 : 1;                   // the products' small parts, then the large ones
   const int lane = threadIdx.x & 63, lr = lane & 15, lq = lane >> 4;
 #pragma unroll 1
   for (int ks = 0; ks < 2; ++ks) {
@@ -94,11 +95,11 @@ __device__ __forceinline__ void pv_tile_careful(f4 (&o)[2][NTR], int key0, int l
           const uint32_t big = half_mask<14>(scale_big(s[pp]));
           h2 hi, lo;
           split_prod(as_h2(x[pp]), as_h2(s[pp] & ~big), hi, lo);
-          a[0][pp] = as_u(hi);
-          a[1][pp] = as_u(lo);
-          split_prod(as_h2(x[pp]), as_h2(s[pp] & big) * h2{(_Float16)0x1p-8f, (_Float16)0x1p-8f}, hi, lo);
+          a[0][pp] = as_u(lo);
           a[2][pp] = as_u(hi);
-          a[3][pp] = as_u(lo) & ~half_mask<15>(non_finite(as_u(hi)));   // (Inf - Inf: the Inf is in hi)
+          split_prod(as_h2(x[pp]), as_h2(s[pp] & big) * h2{(_Float16)0x1p-8f, (_Float16)0x1p-8f}, hi, lo);
+          a[1][pp] = as_u(lo) & ~half_mask<15>(non_finite(as_u(hi)));   // (Inf - Inf: the Inf is in hi)
+          a[3][pp] = as_u(hi);
         } else {
           a[0][pp] = x[pp];
         }
@@ -106,22 +107,29 @@ __device__ __forceinline__ void pv_tile_careful(f4 (&o)[2][NTR], int key0, int l
 #pragma unroll 1
       for (int qi = 0; qi < (masked ? NQ : 1); ++qi) {
         const bool mine = !masked || (lr >> 2) == qi;
-        asm volatile("" ::: "memory");               // (the rows' p16 read again for each query: their registers)
+        asm volatile("" ::: "memory");             // (the rows' p16 read again for each query: their registers)
 #pragma unroll
         for (int nt = 0; nt < NTR; ++nt) {
           const int seen = masked ? lim0 + 4 * nt + qi - k0 : 7;             // the lane's keys 0 .. seen
           uint32_t m[4];
 #pragma unroll
           for (int pp = 0; pp < 4; ++pp) m[pp] = (2 * pp <= seen ? 0xFFFFu : 0u) | (2 * pp + 1 <= seen ? 0xFFFF0000u : 0u);
-          const h8 p = rows(ks, nt);
           const _Float16 f = (_Float16)256.0f;
-          const h8 pb = p * h8{f, f, f, f, f, f, f, f};
-          f4 t = o[mt][nt];
+          h8 p[2];                                 // p16 and p16 * 2^8
+          p[0] = rows(ks, nt);
+          p[1] = p[0] * h8{f, f, f, f, f, f, f, f};
 #pragma unroll
-          for (int i = 0; i < NA; ++i)
-            t = mfma16(__builtin_bit_cast(h8, make_uint4(a[i][0] & m[0], a[i][1] & m[1], a[i][2] & m[2], a[i][3] & m[3])), i < 2 ? p : pb, t);
+          for (int j = 0; j < (VF ? 2 : 1); ++j) { // (the plain products' order)
+            f4 &acc = VF && j == 0 ? l[mt][nt] : o[mt][nt];
+            f4 t = acc;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[mt][nt][i] = mine ? t[i] : o[mt][nt][i];
+            for (int i = 0; i < (VF ? 2 : 1); ++i) {
+              const uint32_t (&b)[4] = a[2 * j + i];
+              t = mfma16(__builtin_bit_cast(h8, make_uint4(b[0] & m[0], b[1] & m[1], b[2] & m[2], b[3] & m[3])), p[i], t);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = mine ? t[i] : acc[i];
+          }
         }
       }
     }

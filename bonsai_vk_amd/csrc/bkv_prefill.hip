@@ -958,45 +958,72 @@ __device__ __forceinline__ void px_gate(const PrefillXArgs &a, size_t row, int d
 // LDS reads. q8_0: one ds_read_b64_tr_b8, and the exact fp16 split of d*b (hi = f16(d*b), lo = d*b -
 // hi) forms two operands shared by the 128 rows. fp16: two ds_read_b64_tr_b16. The ranges' partials are
 // added in a fixed order by prefill_pv_merge_kernel.
-template <int VF, bool PG>
+//
+// Q = kPvQ / 2, for slices of so few queries: 64 rows, each tile's sums from zero and the tiles added in fp64,
+// the small parts of q8_0 products on their own (the fp64 sums of 128 rows would not fit the registers). The
+// matrix cores round every step of an fp32 chain down: given p16, one chain per range is 1.6e-7 (6 queries onto
+// 3000 keys) to 3.3e-7 (14 onto 64000) from 64 bits, this 9.0e-8 and 1.3e-7, decode rows 1.0e-7 and 1.3e-7. Half
+// the rows also take less: 6 onto 3000 11.6 us of 12.2.
+template <int VF, bool PG, int Q>
 __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
-  constexpr int R = kGqa * kPvQ;                   // rows, kPvQ / kPxQ units' worth
+  constexpr int R = kGqa * Q;                      // rows, Q / kPxQ units' worth
   constexpr int NTR = R / 16;                      // MFMA row tiles
   constexpr int RPW = R / 8;                       // rows per wave of the P tile
-  static_assert(RPW == kPxRows, "a wave's rows are one unit");
+  static_assert(kPxRows % RPW == 0, "a wave's rows are a unit or part of one");
+  constexpr int WPU = kPxRows / RPW;               // waves per unit
+  constexpr bool F64 = Q < kPvQ;
   const int n = gridDim.x, b = blockIdx.x;
-  const int nqp = (a.n_q + kPvQ - 1) / kPvQ;
+  const int nqp = (a.n_q + Q - 1) / Q;
   const int wb = (n & 7) == 0 ? (b & 7) * (n >> 3) + (b >> 3) : b;
   const int qb = px_mix(wb % nqp, nqp), sp = (wb / nqp) % a.pv_split, g = wb / (a.pv_split * nqp);
-  const int q0 = a.q_base + kPvQ * qb;             // chunk index of the first query
-  const int nqv = min(kPvQ, a.q_base + a.n_q - q0);
+  const int q0 = a.q_base + Q * qb;                // chunk index of the first query
+  const int nqv = min(Q, a.q_base + a.n_q - q0);
   const uint32_t kend = a.pos0 + (uint32_t)(q0 + nqv);
   const int ntl = (int)((kend + kPfTile - 1) / kPfTile);
   const int t0 = (int)((int64_t)sp * ntl / a.pv_split), t1 = (int)((int64_t)(sp + 1) * ntl / a.pv_split);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lq = lane >> 4;
   __shared__ __attribute__((aligned(16))) float s_pbuf[2 * R * kPfRS / 4];   // P tiles [row][64 keys] fp16
   char *s_p = reinterpret_cast<char *>(s_pbuf);
-  // this thread's probabilities: key pk of a tile, the 16 rows of unit xr (whose scratch holds their e
+  // this thread's probabilities: key pk of a tile, RPW rows of unit xr (whose scratch holds their e
   // up to its own last key kx); the wave's sums in scalar registers
   const int pk = lane;
-  const int xr = kPvQ / kPxQ * qb + w;
+  const int xr = Q / kPxQ * qb + w / WPU;
   const int xq = min(xr, a.nqb - 1);
   const bool pv = kPxQ * xr < a.n_q;
   const uint32_t kx = a.pos0 + (uint32_t)min(a.q_base + kPxQ * xr + kPxQ, a.q_base + a.n_q);
   const size_t xw = (size_t)g * a.nqb + xq;
-  const float *esrc = a.sc + xw * a.ld * kPxRows;
+  const float *esrc = a.sc + (xw * kPxQ + RPW / kGqa * (w % WPU)) * a.ld * kGqa;
   float ssum[RPW], srcp[RPW];
 #pragma unroll
   for (int i = 0; i < RPW; ++i) {
     ssum[i] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
-                                            __builtin_bit_cast(int, a.sums[xw * kPxRows + i])));
+                                            __builtin_bit_cast(int, a.sums[xw * kPxRows + RPW * (w % WPU) + i])));
     srcp[i] = 1.0f / ssum[i];
   }
-  f4 o[2][NTR];
+  f4 o[2][NTR];                                    // (F64: one tile's)
+  f4 ol[2][F64 ? NTR : 1];                         // F64, q8_0: the products' small parts, all tiles
+  auto zero = [&]() {
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < NTR; ++nt) o[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
+  };
+  zero();
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < NTR; ++nt) o[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < (F64 ? NTR : 1); ++nt) ol[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
+  double tot[2][F64 ? NTR : 1][4] = {};
+  auto add = [&]() {
+    if constexpr (F64) {
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NTR; ++nt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) tot[mt][nt][i] += (double)o[mt][nt][i];
+    }
+  };
   // V tiles: three LDS buffers (tile t in buffer t % 3), each of 16 (fp16: 32) blocks of 1 KiB: 16-byte
   // chunk c of row r of block i at 64 (c ^ swizzle(i)) + 16 r, so that the rows one transposed read
   // takes spread over the banks
@@ -1120,8 +1147,7 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
     // this wave's V rows of tile t have landed when at most the loads issued after them are in
     // flight: tile t + 1's register loads (NL) and rows (ND), tile t + 2's register loads (NL)
     constexpr int NL = RPW / 4 + (VF ? 1 : 0);
-    static_assert(2 * NL + ND == 12, "the wait count below");
-    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NL + ND) : "memory");
     // some rows do not see some of the tile's keys, or it is past the range (t1 - 1 again, with p = 0)
     const bool masked = kPfTile * t + kPfTile - 1 > lim0 || t >= t1;
     if (!VF && masked) {                            // the values this wave loaded
@@ -1166,18 +1192,20 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
         }
       }
     }
+    auto rows = [&](int ks, int nt) { return *reinterpret_cast<const h8 *>(pb + (16 * nt + lr) * kPfRS + 2 * (32 * ks + 8 * lq)); };
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
+    for (int nt = 0; nt < NTR; ++nt) {
+      const h8 b0 = rows(0, nt), b1 = rows(1, nt);
 #pragma unroll
-      for (int nt = 0; nt < NTR; ++nt) {
-        const h8 bp = *reinterpret_cast<const h8 *>(pb + (16 * nt + lr) * kPfRS + 2 * (32 * ks + 8 * lq));
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-          o[mt][nt] = mfma16(ah[ks][mt], bp, o[mt][nt]);
-          if constexpr (VF) o[mt][nt] = mfma16(al[ks][mt], bp, o[mt][nt]);
-        }
+      for (int mt = 0; mt < 2; ++mt) {
+        f4 &l = F64 ? ol[mt][F64 ? nt : 0] : o[mt][nt];
+        if constexpr (VF) l = mfma16(al[0][mt], b0, l);
+        o[mt][nt] = mfma16(ah[0][mt], b0, F64 ? f4{0.f, 0.f, 0.f, 0.f} : o[mt][nt]);
+        if constexpr (VF) l = mfma16(al[1][mt], b1, l);
+        o[mt][nt] = mfma16(ah[1][mt], b1, o[mt][nt]);
       }
     }
+    add();
     return false;
   };
   // three register sets and V buffers, each tile's operands requested two tiles ahead (branch-free
@@ -1213,10 +1241,16 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
       probs(in[0], s_p, vsk);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       lds_barrier();
+      auto &l = [&]() -> f4 (&)[2][NTR] {
+        if constexpr (F64) return ol;
+        else return o;
+      }();
+      if constexpr (F64) zero();
       pv_tile_careful<VF, NTR, kPxQ>(
-          o, kPfTile * t, lim0, kPfTile * t + kPfTile - 1 > lim0,
+          o, l, kPfTile * t, lim0, kPfTile * t + kPfTile - 1 > lim0,
           [&](int ks, int mt, uint32_t (&x)[4], uint32_t (&s)[4]) { operand(vread(t, ks, mt), ks, vsk, x, s); },
           [&](int ks, int nt) { return *reinterpret_cast<const h8 *>(s_p + (16 * nt + lr) * kPfRS + 2 * (32 * ks + 8 * lq)); });
+      add();
     }
   }
   // lane l holds out^T[dim 32 w + 16 mt + 4(l/16) + r][row 16 nt + l%16] in o[mt][nt][r]: the range's
@@ -1231,25 +1265,34 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
       const int d = 32 * w + 16 * mt + 4 * lq;
-      const float4 v = make_float4(o[mt][nt][0], o[mt][nt][1], o[mt][nt][2], o[mt][nt][3]);
+      float4 v = make_float4(o[mt][nt][0], o[mt][nt][1], o[mt][nt][2], o[mt][nt][3]);
+      if constexpr (F64) {
+        double x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = tot[mt][nt][i] + (double)ol[mt][nt][i];
+        v = make_float4((float)x[0], (float)x[1], (float)x[2], (float)x[3]);
+      }
       *reinterpret_cast<float4 *>(part + row * kHd + d) = v;
       if (whole && a.gate) px_gate(a, (size_t)a.q_base * a.nh + row, d, v);
     }
   }
 }
 
-// out = the key ranges' partials added in range order, and the gate
+// out = the key ranges' partials (8 requested together and added pairwise, the eights in fp64), and the gate
 __global__ __launch_bounds__(256) void prefill_pv_merge_kernel(PrefillXArgs a) {
   const size_t n4 = (size_t)a.n_q * a.nh * (kHd / 4);
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n4) return;
-  const float4 *pp = reinterpret_cast<const float4 *>(a.part) + i;
-  float4 v = pp[0];
-#pragma unroll 8
-  for (int s = 1; s < a.pv_split; ++s) {
-    const float4 y = pp[(size_t)s * n4];
-    v = make_float4(v.x + y.x, v.y + y.y, v.z + y.z, v.w + y.w);
+  const f4 *pp = reinterpret_cast<const f4 *>(a.part) + i;
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  for (int s = 0; s < a.pv_split; s += 8) {
+    f4 y[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) y[u] = s + u < a.pv_split ? pp[(size_t)(s + u) * n4] : f4{0.f, 0.f, 0.f, 0.f};
+    const f4 t = ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7]));
+    s0 += (double)t[0]; s1 += (double)t[1]; s2 += (double)t[2]; s3 += (double)t[3];
   }
+  const float4 v = make_float4((float)s0, (float)s1, (float)s2, (float)s3);
   const size_t grow = (size_t)a.q_base * a.nh + i / (kHd / 4);   // row of the whole chunk
   const int d = 4 * (int)(i % (kHd / 4));
   *reinterpret_cast<float4 *>(a.out + grow * kHd + d) = v;
@@ -1317,18 +1360,25 @@ hipError_t launch_prefill_exact(PrefillXArgs a, int kf, int vf, hipStream_t st) 
   else hipLaunchKernelGGL(prefill_sum_kernel<4>, dim3(units), dim3(256), 0, st, a);
   // PV: one workgroup per CU, 3 us per tile and 8 for the rest (512 onto 8192: 104 us in one round; 48
   // onto 6000: 17 us in one round, 28 in two)
-  const int items = a.nkv * ((a.n_q + kPvQ - 1) / kPvQ);
+  const bool few = a.n_q <= kPvQ / 2;
+  const int items = few ? a.nkv : a.nkv * ((a.n_q + kPvQ - 1) / kPvQ);
   // (the merge reads a range's partials at about 4 TB/s)
   a.pv_split = px_ranges(items, (kmax + kPfTile - 1) / kPfTile, 256, 3000, 8000, (int64_t)a.n_q * a.nh * kHd * 4 / 4000,
                          kPvSplit * kPxSlice / a.n_q);
   const dim3 pgrid(items * a.pv_split);
+#define BKV_LAUNCH_PV(VF, Q)                                                                             \
+  do {                                                                                                   \
+    if (pg) hipLaunchKernelGGL((prefill_pv64_kernel<VF, true, Q>), pgrid, dim3(512), 0, st, a);          \
+    else hipLaunchKernelGGL((prefill_pv64_kernel<VF, false, Q>), pgrid, dim3(512), 0, st, a);            \
+  } while (0)
   if (vf == BKV_Q8_0) {
-    if (pg) hipLaunchKernelGGL((prefill_pv64_kernel<1, true>), pgrid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((prefill_pv64_kernel<1, false>), pgrid, dim3(512), 0, st, a);
+    if (few) BKV_LAUNCH_PV(1, kPvQ / 2);
+    else BKV_LAUNCH_PV(1, kPvQ);
   } else {
-    if (pg) hipLaunchKernelGGL((prefill_pv64_kernel<0, true>), pgrid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((prefill_pv64_kernel<0, false>), pgrid, dim3(512), 0, st, a);
+    if (few) BKV_LAUNCH_PV(0, kPvQ / 2);
+    else BKV_LAUNCH_PV(0, kPvQ);
   }
+#undef BKV_LAUNCH_PV
   if (a.pv_split == 1) return hipGetLastError();
   const size_t n4 = (size_t)a.n_q * a.nh * (kHd / 4);
   hipLaunchKernelGGL(prefill_pv_merge_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, a);

@@ -7,8 +7,11 @@
 // e in key order (the reference's serial fp32 sum, attn_vk.h:175-189), p16 = f16(e / sum) goes to LDS and
 // the PV runs on the matrix cores from V tiles that direct-to-LDS loads brought in behind the scores.
 // What bounds it: a chain of latencies (K rows, scores, exps, the serial sum at about 5 ns per key, V
-// tiles), so the limit of 512 keys is where the stream kernel's wider spread of keys takes over.
-// Scores, e, sums and p16 are bit-identical to the other kernels'; only the PV sum's order differs.
+// tiles); past 384 keys with q8_0 V (448 with fp16 V and pages) a decode is faster where the stream or
+// resident kernel spreads the keys wider (short_decode_keys). Chunks take it to kShortKeys.
+// Scores, e, sums and p16 are bit-identical to the other kernels'; the PV sum's order differs. Its error
+// given p16 (2-norm, q8_0 V) is 6.6e-8 at 64 keys, 8.3e-8 at 300, 8.8e-8 at 384 (the stream kernel's 6.9e-8,
+// 8.5e-8, 8.4e-8; one fp32 chain over all products 8.8e-8, 1.7e-7, 1.9e-7).
 #include <type_traits>
 
 #include "bkv_device.h"
@@ -53,9 +56,8 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
   __shared__ __attribute__((aligned(16))) float s_gate[NR == 4 ? NR * kHd : 4];  // 1 / (1 + exp(-gate))
   __shared__ float s_ex[16], s_red[8][NR], s_sum[NR];
   __shared__ int s_lt[kGqa];
-  __shared__ unsigned s_flags, s_wide;
-  __shared__ __attribute__((aligned(8))) uint8_t s_big[8];   // (q8_0 V) tile t has a scale past the plain products
-  if (tid == 0) { s_flags = 0u; s_wide = 0u; }
+  __shared__ unsigned s_flags, s_wide, s_big;      // (s_big: a V scale past the plain products)
+  if (tid == 0) { s_flags = 0u; s_wide = 0u; s_big = 0u; }
   if (tid < 32) s_t2[tid] = kExp2Tab[tid];
   static_assert(16 * kShPS >= kQ8fUnit * 16 && 16 * kShPS >= kHd * 16 * 4 && 16 * kShPS >= kLimBytes, "q16 operands in s_p");
   lds_barrier();
@@ -355,11 +357,12 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
                    : "memory", "m0");
     }
   };
+  const int sw = (w + 7) & 7;                      // the tile whose scale rows this wave takes (wave 0: the eighth)
   if constexpr (VF) {
-    if (w < nt) {
-      const uint8_t *src = a.L.vs + krow(64 * w + lane) * kScaleRowBytes;
+    if (sw < nt) {
+      const uint8_t *src = a.L.vs + krow(64 * sw + lane) * kScaleRowBytes;
       asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src),
-                   "s"(__builtin_amdgcn_readfirstlane(lds_addr(s_vs) + 1024u * (uint32_t)w)) : "memory", "m0");
+                   "s"(__builtin_amdgcn_readfirstlane(lds_addr(s_vs) + 1024u * (uint32_t)sw)) : "memory", "m0");
     }
   }
   for (int t = 0; t < min(nt, NB); ++t) dma_tile(t);
@@ -433,6 +436,14 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
       }
     }
   }
+  if (VF && (w > 0 || nt == 8)) {
+    // Beside the serial sums: the scale rows have landed. (The appended token's, also for the padding after it:
+    // those entries were loaded from its slot, which may have held anything, and p = 0 times a NaN scale is NaN.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (append && sw == (kend - 1) >> 6 && lane >= ((kend - 1) & 63)) s_vs[64 * sw + lane] = s_row[1][16];
+    const uint4 s = s_vs[64 * sw + lane];
+    if (sw < nt && __any((scale_big(s.x) | scale_big(s.y) | scale_big(s.z) | scale_big(s.w)) != 0u)) s_big = 1u;
+  }
   if (NR == 4 && a.gate && w > 0) {
     // the gate's factors beside the serial sums (fp64 exps and divisions: 2 us behind the PV)
     for (int i = tid - 64; i < NR * kHd; i += kShNT - 64)
@@ -458,122 +469,160 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
                            8 * (lane & 1));
     }
   }
-  f4 o[2][1] = {{f4{0.f, 0.f, 0.f, 0.f}}, {f4{0.f, 0.f, 0.f, 0.f}}};
-  unsigned long big = 0;                           // byte t: s_big
-  for (int t = 0; t < nt; ++t) {
-    // The first NB tiles have landed at t = 0. Tile t + NB - 1 goes into tile t - 1's buffer once every wave
-    // has read that one; later tiles are waited for in order, the younger ones' loads left in flight.
-    if (t == 0) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      // (the appended token's scales, also for the padding after it: those entries were loaded from its slot,
-      // which may have held anything, and p = 0 times a NaN scale is NaN)
-      if (VF && append && w == (kend - 1) >> 6 && lane >= ((kend - 1) & 63)) s_vs[64 * w + lane] = s_row[1][16];
-      if (VF && w < nt) {
-        const uint4 s = s_vs[64 * w + lane];
-        const bool b = __any((scale_big(s.x) | scale_big(s.y) | scale_big(s.z) | scale_big(s.w)) != 0u);
-        if (lane == 0) s_big[w] = b;
-      }
-      lds_barrier();                               // every wave's rows, and p16
-      if (VF) big = *reinterpret_cast<const unsigned long *>(s_big);
-    } else if (nt > NB) {
-      if (t >= NB) {
-        if (t + 1 >= nt) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ND) : "memory");
-      }
-      lds_barrier();
-      if (t + NB - 1 < nt) dma_tile(t + NB - 1);
-    }
-    char *vt = s_v[t % NB];
-    if (append && t == nt - 1) {                   // the appended row, this wave's dims, over its loaded copy
-      const int r = (kend - 1) & 63;
-      if constexpr (VF) {
-        const int i = r >> 2;
-        if (lane < 2)
-          *reinterpret_cast<uint4 *>(vt + 1024 * i + 64 * ((2 * w + lane) ^ (i & 3)) + 16 * (r & 3)) = s_row[1][2 * w + lane];
-      } else {                                     // (and over the padding's copies: see the scales)
-        const int c = 4 * (w & 3) + (lane & 3);
-        for (int rr = r + (lane >> 2); rr < 64; rr += 16) {
-          const int i = rr >> 2;
-          *reinterpret_cast<uint4 *>(vt + 1024 * (i + 16 * (w >> 2)) + 64 * (c ^ (2 * ((i >> 1) & 3))) + 16 * (rr & 3)) =
-              s_row[1][4 * w + (lane & 3)];
-        }
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
-    const uint32_t vb = vbase + (uint32_t)VB * (uint32_t)(t % NB);
-    const int lim0 = (int)a.pos0 + q0;             // the first query's last key
-    const bool masked = 64 * t + 63 > lim0;        // some rows do not see some of the tile's keys
-    auto rows = [&](int ks, int) { return *reinterpret_cast<const h8 *>(s_p + lr * kShPS + 2 * (64 * t + 32 * ks + 8 * lq)); };
-    // the V operand in pairs of keys (see pv_tile_careful)
-    auto ops = [&](int ks, int mt, uint32_t (&x)[4], uint32_t (&s)[4]) {
-      if constexpr (VF) {
-        const uint16_t *vs = reinterpret_cast<const uint16_t *>(&s_vs[64 * t + 32 * ks + 8 * lq]) + w;
-        const v2i_t bv = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-            (__attribute__((address_space(3))) v2i_t *)(uintptr_t)((vb + vrd[ks]) ^ (uint32_t)(64 * (2 * w + mt))));
-        constexpr uint32_t kSel[4] = {0x0C010C00u, 0x0C030C02u, 0x0C050C04u, 0x0C070C06u};
-#pragma unroll
-        for (int pp = 0; pp < 4; ++pp) {
-          const uint32_t bw = __builtin_amdgcn_perm((uint32_t)bv.y, (uint32_t)bv.x, kSel[pp]) ^ 0x64806480u;
-          x[pp] = as_u(as_h2(bw) - h2{(_Float16)1152.0f, (_Float16)1152.0f});
-          s[pp] = (uint32_t)vs[16 * pp] | ((uint32_t)vs[16 * pp + 8] << 16);
-        }
-      } else {
-        const uint32_t ad = (vb + vrd[ks]) ^ (uint32_t)(128 * (2 * (w & 3) + mt));
-        const v4s_t r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)ad);
-        const v4s_t r1 =
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)(ad + 1024u));
-        const uint4 v = __builtin_bit_cast(uint4, (v8s_t){r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]});
-        x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
-      }
-    };
-    uint32_t x[2][2][4], s[2][4];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt) ops(ks, mt, x[ks][mt], s[ks]);
-    bool careful = false;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the first NB tiles have landed
+  lds_barrier();                                   // every wave's rows, and p16
+  const int lim0 = (int)a.pos0 + q0;               // the first query's last key
+  auto rows = [&](int t, int ks) { return *reinterpret_cast<const h8 *>(s_p + lr * kShPS + 2 * (64 * t + 32 * ks + 8 * lq)); };
+  // the V operand in pairs of keys (see pv_tile_careful)
+  auto ops = [&](int t, int ks, int mt, uint32_t (&x)[4], uint32_t (&s)[4]) {
+    const uint32_t vb = vbase + (uint32_t)VB * (uint32_t)(t % NB) + vrd[ks];
     if constexpr (VF) {
-      careful = (__builtin_amdgcn_readfirstlane((int)(big >> (8 * t))) & 0xFF) != 0;
-    } else if (masked) {
-      uint32_t nf = 0;
+      const uint16_t *vs = reinterpret_cast<const uint16_t *>(&s_vs[64 * t + 32 * ks + 8 * lq]) + w;
+      const v2i_t bv = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+          (__attribute__((address_space(3))) v2i_t *)(uintptr_t)(vb ^ (uint32_t)(64 * (2 * w + mt))));
+      constexpr uint32_t kSel[4] = {0x0C010C00u, 0x0C030C02u, 0x0C050C04u, 0x0C070C06u};
 #pragma unroll
-      for (int i = 0; i < 16; ++i) nf |= non_finite(x[i >> 3][(i >> 2) & 1][i & 3]);
-      careful = __any(nf != 0u);
-    }
-    if (careful) {
-      pv_tile_careful<VF, 1, NQ>(o, 64 * t, lim0, masked, ops, rows);
+      for (int pp = 0; pp < 4; ++pp) {
+        const uint32_t bw = __builtin_amdgcn_perm((uint32_t)bv.y, (uint32_t)bv.x, kSel[pp]) ^ 0x64806480u;
+        x[pp] = as_u(as_h2(bw) - h2{(_Float16)1152.0f, (_Float16)1152.0f});
+        s[pp] = (uint32_t)vs[16 * pp] | ((uint32_t)vs[16 * pp + 8] << 16);
+      }
     } else {
+      const uint32_t ad = vb ^ (uint32_t)(128 * (2 * (w & 3) + mt));
+      const v4s_t r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)ad);
+      const v4s_t r1 =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t *)(uintptr_t)(ad + 1024u));
+      const uint4 v = __builtin_bit_cast(uint4, (v8s_t){r0[0], r0[1], r0[2], r0[3], r1[0], r1[1], r1[2], r1[3]});
+      x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+    }
+  };
+  // Chains per value by tile (mod NS) and key half, and the small parts of q8_0 products on their own: the
+  // matrix cores round every step of a chain down (see the header).
+  constexpr int NS = NR == 4 ? 2 : 3;
+  f4 zh[NS][2][2] = {}, zl[2][1] = {};             // [tile mod NS][key half][mt]; [mt]
+  auto careful = [&](int t) {
+    f4 z[2][1] = {{zh[0][0][0]}, {zh[0][0][1]}};
+    uint32_t x[2][2][4], s[2][4];                  // (requested together)
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        const h8 bp = rows(ks, 0);
+    for (int i = 0; i < 4; ++i) ops(t, i >> 1, i & 1, x[i >> 1][i & 1], s[i >> 1]);
+    pv_tile_careful<VF, 1, NQ>(
+        z, zl, 64 * t, lim0, 64 * t + 63 > lim0,
+        [&](int ks, int mt, uint32_t (&xk)[4], uint32_t (&sk)[4]) {
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-          const uint32_t (&xk)[4] = x[ks][mt];
-          if constexpr (VF) {
-            uint32_t hw[4], lw[4];
-#pragma unroll
-            for (int pp = 0; pp < 4; ++pp) {
-              h2 hi, lo;
-              split_prod(as_h2(xk[pp]), as_h2(s[ks][pp]), hi, lo);
-              hw[pp] = as_u(hi);
-              lw[pp] = as_u(lo);
-            }
-            o[mt][0] = mfma16(__builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3])), bp, o[mt][0]);
-            o[mt][0] = mfma16(__builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3])), bp, o[mt][0]);
-          } else {
-            o[mt][0] = mfma16(__builtin_bit_cast(h8, make_uint4(xk[0], xk[1], xk[2], xk[3])), bp, o[mt][0]);
+          for (int i = 0; i < 4; ++i) {
+            xk[i] = ks ? x[1][mt][i] : x[0][mt][i];
+            sk[i] = ks ? s[1][i] : s[0][i];
+          }
+        },
+        [&](int ks, int) { return rows(t, ks); });
+    zh[0][0][0] = z[0][0];
+    zh[0][0][1] = z[1][0];
+  };
+  unsigned later = 0;                              // fp16 V: tiles that need pv_tile_careful (of this wave's dims)
+  // (CAREFUL: q8_0 V with a scale past the plain products, a loop of its own so that the other stays small)
+  auto loop = [&](auto mode) {
+    constexpr bool CAREFUL = decltype(mode)::value;
+    for (int t = 0; t < nt; ++t) {
+      // Tile t + NB - 1 goes into tile t - 1's buffer once every wave has read that one; later tiles are waited
+      // for in order, the younger ones' loads left in flight.
+      if (t > 0 && nt > NB) {
+        if (t >= NB) {
+          if (t + 1 >= nt) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ND) : "memory");
+        }
+        lds_barrier();
+        if (t + NB - 1 < nt) dma_tile(t + NB - 1);
+      }
+      char *vt = s_v[t % NB];
+      if (append && t == nt - 1) {                 // the appended row, this wave's dims, over its loaded copy
+        const int r = (kend - 1) & 63;
+        if constexpr (VF) {
+          const int i = r >> 2;
+          if (lane < 2)
+            *reinterpret_cast<uint4 *>(vt + 1024 * i + 64 * ((2 * w + lane) ^ (i & 3)) + 16 * (r & 3)) = s_row[1][2 * w + lane];
+        } else {                                   // (and over the padding's copies: see the scales)
+          const int c = 4 * (w & 3) + (lane & 3);
+          for (int rr = r + (lane >> 2); rr < 64; rr += 16) {
+            const int i = rr >> 2;
+            *reinterpret_cast<uint4 *>(vt + 1024 * (i + 16 * (w >> 2)) + 64 * (c ^ (2 * ((i >> 1) & 3))) + 16 * (rr & 3)) =
+                s_row[1][4 * w + (lane & 3)];
           }
         }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+      if constexpr (CAREFUL) {
+        careful(t);
+      } else {
+        uint32_t x[2][2][4], s[2][4];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt) ops(t, ks, mt, x[ks][mt], s[ks]);
+        const h8 bp[2] = {rows(t, 0), rows(t, 1)};
+        bool plain = true;
+        if (!VF && 64 * t + 63 > lim0) {           // some rows do not see some of the tile's keys
+          uint32_t nf = 0;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) nf |= non_finite(x[i >> 3][(i >> 2) & 1][i & 3]);
+          plain = !__any(nf != 0u);
+          if (!plain) later |= 1u << t;
+        }
+        if (plain) {
+          h8 hi[2][2];
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+              const uint32_t (&xk)[4] = x[ks][mt];
+              if constexpr (VF) {
+                uint32_t hw[4], lw[4];
+#pragma unroll
+                for (int pp = 0; pp < 4; ++pp) {
+                  h2 h, l;
+                  split_prod(as_h2(xk[pp]), as_h2(s[ks][pp]), h, l);
+                  hw[pp] = as_u(h);
+                  lw[pp] = as_u(l);
+                }
+                hi[ks][mt] = __builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3]));
+                zl[mt][0] = mfma16(__builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3])), bp[ks], zl[mt][0]);
+              } else {
+                hi[ks][mt] = __builtin_bit_cast(h8, make_uint4(xk[0], xk[1], xk[2], xk[3]));
+              }
+            }
+          }
+          auto step = [&](f4 (&zp)[2][2]) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+              for (int mt = 0; mt < 2; ++mt) zp[ks][mt] = mfma16(hi[ks][mt], bp[ks], zp[ks][mt]);
+          };
+          const int ts = t % NS;
+          if (ts == 0) step(zh[0]);
+          else if (ts == 1) step(zh[1]);
+          else step(zh[NS - 1]);
+        }
       }
     }
+  };
+  if (__builtin_expect(VF && s_big != 0u, 0)) loop(std::integral_constant<bool, VF != 0>{});
+  else loop(std::false_type{});
+  if constexpr (!VF)                               // (the last two tiles at most, still in their buffers)
+    for (int t = 0; later != 0u; ++t, later >>= 1)
+      if (later & 1u) careful(t);
+  f4 o[2];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt) {
+    o[mt] = (zh[0][0][mt] + zh[0][1][mt]) + (zh[1][0][mt] + zh[1][1][mt]);
+    if constexpr (NS == 3) zl[mt][0] = (zh[2][0][mt] + zh[2][1][mt]) + zl[mt][0];
+    o[mt] = o[mt] + zl[mt][0];
   }
-  // lane l holds out^T[dim 32 w + 16 mt + 4 lq + i][row lr] in o[mt][0][i]
+  // lane l holds out^T[dim 32 w + 16 mt + 4 lq + i][row lr] in o[mt][i]
   if (lr < NR && (lr >> 2) < nqv) {
     const size_t row = (size_t)(q0 + (lr >> 2)) * a.nh + g * kGqa + (lr & 3);
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
       const int d = 32 * w + 16 * mt + 4 * lq;
-      const float4 v = make_float4(o[mt][0][0], o[mt][0][1], o[mt][0][2], o[mt][0][3]);
+      const float4 v = make_float4(o[mt][0], o[mt][1], o[mt][2], o[mt][3]);
       *reinterpret_cast<float4 *>(a.out + row * kHd + d) = v;
       if (a.gate) {
         float4 f;

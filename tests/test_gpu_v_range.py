@@ -71,8 +71,9 @@ def test_q8v_past_fp16(pos0, n, kind, kf):
 @pytest.mark.parametrize("pos0,n", [s for s in SHAPES if s[1] > 1] + [(100, 40)])
 def test_later_tokens_non_finite_v(pos0, n, what, kf, vf):
     """A token whose V is stored as Inf or NaN (also a value past the format's range) in the last token of a
-    chunk and in one before it: the queries before each are what they are without it, bit for bit, and the
-    others are finite, Inf and NaN where the oracle is."""
+    chunk and in one before it: the queries before each are what they are without it (up to the order of the PV
+    sum: at most m steps, each within 2^-23 of a partial sum that the row's largest |v| bounds), and the others
+    are finite, Inf and NaN where the oracle is."""
     say(f"non-finite V: pos0={pos0} n={n} {what} kf={kf} vf={vf}")
     m = pos0 + n
     v = oracle.synth_kv(m, 4, 256, 9, 0, outliers=3)[1]
@@ -83,7 +84,7 @@ def test_later_tokens_non_finite_v(pos0, n, what, kf, vf):
     plain, _ = both(*filled(pos0, n, kf, vf, v), pos0, n)
     dev, host = filled(pos0, n, kf, vf, bad)
     out, want = both(dev, host, pos0, n)
-    assert np.array_equal(out[:first - pos0], plain[:first - pos0])
+    assert np.abs(out[:first - pos0] - plain[:first - pos0]).max(initial=0.0) <= m * 2.0 ** -23 * np.abs(v).max()
     assert np.array_equal(np.isnan(out), np.isnan(want)) and np.array_equal(np.isinf(out), np.isinf(want))
     ok = np.isfinite(want)
     assert np.array_equal(np.sign(out[np.isinf(want)]), np.sign(want[np.isinf(want)]))

@@ -506,6 +506,16 @@ static bool px_worthwhile(int n_q, int64_t keys) {
   return n_q >= kPxMinQ || (n_q > 1 && n_q * (170000 + 4 * keys) > 260000 + 62 * keys);
 }
 
+// Whether a chunk of a short context runs in the short kernel, whose workgroups (4 queries of a KV group) fill
+// the chip in rounds of 256, or in the chunk kernels, whose time is nearly flat: up to about 860,000
+// workgroup * (first + last key + 320). us, short / chunk kernels, q8_0 and fp16 K + V: 200 queries onto 100 keys,
+// 16 KV heads (576,000) 47.7 / 53.4, 68.4 / 68.8; 512 onto none, 8 heads (850,000) 62.3 / 70.0, 85.9 / 87.7; 330
+// onto none, 16 heads (863,000) 73.0 / 62.2, 103.7 / 77.7; 200 onto 300, 16 heads (896,000) 76.8 / 71.6,
+// 102.4 / 89.5; 512 onto none, 32 heads 232 / 174, 323 / 230.
+static bool short_chunk(int nkv, int64_t pos0, int64_t n_q) {
+  return n_q < kPxMinQ || nkv * cdiv(n_q, kPxQ) * (2 * pos0 + n_q + 320) <= 860000;
+}
+
 static int prefill_common(const bkv_cache_desc *d, int layer, uint32_t pos0, int n_q,
                           const float *q, const float *gate, float *out, float *out_gated,
                           void *workspace, size_t ws_bytes, hipStream_t stream, int qs, int gs) {
@@ -522,7 +532,7 @@ static int prefill_common(const bkv_cache_desc *d, int layer, uint32_t pos0, int
   if (!workspace) return BKV_EWORKSPACE;
   if (((uintptr_t)workspace & 255u) != 0) return BKV_EALIGN;
   const size_t base = prefill_base(d);
-  if (!prefill_mfma_requested() && n_q > 1 && (int64_t)pos0 + n_q <= kShortKeys) {
+  if (!prefill_mfma_requested() && n_q > 1 && (int64_t)pos0 + n_q <= kShortKeys && short_chunk(d->nkv, pos0, n_q)) {
     // a short context: one launch, 4 queries per workgroup (the workspace is asked for all the same, so
     // that a caller meets its size at the first chunk and not at a later one)
     const size_t need = n_q >= kPxMinQ ? px_layout(d->nh, d->nkv, (int64_t)pos0 + n_q, kPxSlice, base).total

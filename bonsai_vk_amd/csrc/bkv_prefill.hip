@@ -981,7 +981,8 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
   const uint32_t kend = a.pos0 + (uint32_t)(q0 + nqv);
   const int ntl = (int)((kend + kPfTile - 1) / kPfTile);
   const int t0 = (int)((int64_t)sp * ntl / a.pv_split), t1 = (int)((int64_t)(sp + 1) * ntl / a.pv_split);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lq = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   __shared__ __attribute__((aligned(16))) float s_pbuf[2 * R * kPfRS / 4];   // P tiles [row][64 keys] fp16
   char *s_p = reinterpret_cast<char *>(s_pbuf);
   // this thread's probabilities: key pk of a tile, RPW rows of unit xr (whose scratch holds their e
@@ -994,12 +995,6 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
   const size_t xw = (size_t)g * a.nqb + xq;
   const float *esrc = a.sc + (xw * kPxQ + RPW / kGqa * (w % WPU)) * a.ld * kGqa;
   float ssum[RPW], srcp[RPW];
-#pragma unroll
-  for (int i = 0; i < RPW; ++i) {
-    ssum[i] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
-                                            __builtin_bit_cast(int, a.sums[xw * kPxRows + RPW * (w % WPU) + i])));
-    srcp[i] = 1.0f / ssum[i];
-  }
   f4 o[2][NTR];                                    // (F64: one tile's)
   f4 ol[2][F64 ? NTR : 1];                         // F64, q8_0: the products' small parts, all tiles
   auto zero = [&]() {
@@ -1051,14 +1046,14 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
     bool live;
     uint32_t vs;                                    // the block scale of key 32 (l%16 / 8) + 8 lq + l%8
   };
-  // tiles past t1 (the loop runs whole groups of three) load tile t1 - 1 again and add nothing
+  // (past t1, ahead of the loop's end: tile t1 - 1 again)
   auto load_tile = [&](int tt, PvIn &in) {
     const int t = min(tt, t1 - 1);
     const uint32_t j = (uint32_t)(t * kPfTile + pk);
     const float *src = esrc + (size_t)min(j, kx - 1) * kGqa;
 #pragma unroll
     for (int i = 0; i < RPW / 4; ++i) in.en[i] = ld_sc4(src + (size_t)i * a.ld * kGqa);
-    in.live = pv && j < kx && tt < t1;
+    in.live = pv && j < kx;
     if constexpr (VF) {
       // one scale load per lane: lane l%16 of each 16-lane row loads key (l%16 / 8, l%8)'s, and the row
       // shares them by DPP broadcasts in the tile
@@ -1148,8 +1143,7 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
     // flight: tile t + 1's register loads (NL) and rows (ND), tile t + 2's register loads (NL)
     constexpr int NL = RPW / 4 + (VF ? 1 : 0);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NL + ND) : "memory");
-    // some rows do not see some of the tile's keys, or it is past the range (t1 - 1 again, with p = 0)
-    const bool masked = kPfTile * t + kPfTile - 1 > lim0 || t >= t1;
+    const bool masked = kPfTile * t + kPfTile - 1 > lim0;   // some rows do not see some of the tile's keys
     if (!VF && masked) {                            // the values this wave loaded
       uint32_t nf = 0;
 #pragma unroll
@@ -1208,8 +1202,8 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
     add();
     return false;
   };
-  // three register sets and V buffers, each tile's operands requested two tiles ahead (branch-free
-  // groups of three, so that the compiler's wait counting keeps the two younger tiles' loads in
+  // three register sets and V buffers, each tile's operands requested two tiles ahead (groups of three
+  // without joining branches, so that the compiler's wait counting keeps the two younger tiles' loads in
   // flight); the V rows of tile t + 2 go out once every wave has passed tile t's barrier
   if (t0 < t1) {
     PvIn in[3];
@@ -1218,9 +1212,17 @@ __global__ __launch_bounds__(512, 1) void prefill_pv64_kernel(PrefillXArgs a) {
     dma_tile(t0);
     load_tile(t0 + 1, in[1]);
     dma_tile(t0 + 1);
+    // (the sums behind the first tiles' loads, which do not need them)
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+      ssum[i] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+                                              __builtin_bit_cast(int, a.sums[xw * kPxRows + RPW * (w % WPU) + i])));
+      srcp[i] = 1.0f / ssum[i];
+    }
     for (int t = t0; t < t1; t += 3) {
 #pragma unroll
       for (int u = 0; u < 3; ++u) {
+        if (u > 0 && t + u >= t1) break;
         load_tile(t + u + 2, in[(u + 2) % 3]);
         __builtin_amdgcn_sched_barrier(0);
         if (tile(t + u, in[u])) {                   // (the same in every wave)
@@ -1342,10 +1344,20 @@ hipError_t launch_prefill_exact(PrefillXArgs a, int kf, int vf, hipStream_t st) 
     // its matrix cores: 24 us for a 256-key tile of each. (300 queries onto 2000 keys: 67 us with every
     // tile a workgroup, 1000 onto none: 75 us, 82-84 with fewer workgroups; 512 onto 8192: 352 us, 392
     // with one unit and two sets of keys per wave.)
-    const int items = a.nkv * ((a.nqb + 1) / 2);
-    a.ksplit = px_ranges(items, (kmax + kPxTile16 - 1) / kPxTile16, 1024, 24000, 2000, 0, mxmost);
+    // One unit where the rounds of 256 workgroups then come out shorter (6.8 us a tile, 12.2 with two): 256 onto
+    // 500 (768 workgroups of one tile, not 384) 52.3 us for the call, 56.3 with two; 100 onto 1000 47.3, 55.2; 20
+    // onto 6000 67.2, 75.3; but 256 onto 700 61.6, 60.6; 1000 onto none 145, 132.
+    const int64_t tiles = (kmax + kPxTile16 - 1) / kPxTile16;
+    int items = 0;
+    auto plan = [&](int nu, int64_t tile) {
+      items = a.nkv * ((a.nqb + nu - 1) / nu);
+      a.ksplit = px_ranges(items, tiles, 1024, 24000, 2000, 0, mxmost);
+      return ((int64_t)items * a.ksplit + 255) / 256 * ((tiles + a.ksplit - 1) / a.ksplit) * tile;
+    };
+    const bool one = a.nqb == 1 || (units <= 256 && plan(1, 6800) < plan(2, 12200));
+    plan(one ? 1 : 2, 0);
     const dim3 grid(items * a.ksplit);
-    if (a.nqb == 1) {
+    if (one) {
       if (pg) hipLaunchKernelGGL((prefill_score_f16_kernel<1, true>), grid, dim3(256), 0, st, a);
       else hipLaunchKernelGGL((prefill_score_f16_kernel<1, false>), grid, dim3(256), 0, st, a);
     } else {
@@ -1359,11 +1371,12 @@ hipError_t launch_prefill_exact(PrefillXArgs a, int kf, int vf, hipStream_t st) 
   if (units <= 256) hipLaunchKernelGGL(prefill_sum_kernel<8>, dim3(units), dim3(512), 0, st, a);
   else hipLaunchKernelGGL(prefill_sum_kernel<4>, dim3(units), dim3(256), 0, st, a);
   // PV: one workgroup per CU, 3 us per tile and 8 for the rest (512 onto 8192: 104 us in one round; 48
-  // onto 6000: 17 us in one round, 28 in two)
+  // onto 6000: 17 us in one round, 28 in two; 128 onto 500, fp16 V: 10 ranges of one tile 44.4 us for the
+  // call, 4 of three 39.8)
   const bool few = a.n_q <= kPvQ / 2;
   const int items = few ? a.nkv : a.nkv * ((a.n_q + kPvQ - 1) / kPvQ);
-  // (the merge reads a range's partials at about 4 TB/s)
-  a.pv_split = px_ranges(items, (kmax + kPfTile - 1) / kPfTile, 256, 3000, 8000, (int64_t)a.n_q * a.nh * kHd * 4 / 4000,
+  // (a range's partials are written and read at about 4 TB/s)
+  a.pv_split = px_ranges(items, (kmax + kPfTile - 1) / kPfTile, 256, 3000, 8000, (int64_t)a.n_q * a.nh * kHd * 8 / 4000,
                          kPvSplit * kPxSlice / a.n_q);
   const dim3 pgrid(items * a.pv_split);
 #define BKV_LAUNCH_PV(VF, Q)                                                                             \

@@ -119,3 +119,22 @@ def test_short_decode_step_into_unwritten_slots(kf, vf, n):
         outs.append(c.decode_step(0, n - 1, k[n - 1:], v[n - 1:], q)[0])
     torch.cuda.synchronize()
     assert bool(torch.isfinite(outs[0]).all()) and torch.equal(outs[0], outs[1])
+
+
+# 16 KV heads: a chunk of a short context in the short kernel, and one of so many workgroups that it leaves it
+@pytest.mark.parametrize("kf,vf", [(BKV_Q8_0, BKV_Q8_0), (BKV_F16, BKV_F16)])
+@pytest.mark.parametrize("pos0,n", [(300, 100), (300, 200), (0, 331)])
+def test_short_chunk_of_many_kv_heads(kf, vf, pos0, n):
+    say(f"short chunk, 16 KV heads kf={kf} vf={vf} pos0={pos0} n={n}")
+    m = pos0 + n
+    dev = KvCache(n_layers=1, nh=64, nkv=16, cap=m, k_fmt=kf, v_fmt=vf)
+    host = oracle.HostCache(n_layers=1, nh=64, nkv=16, cap=m, k_fmt=kf, v_fmt=vf)
+    k, v = oracle.synth_kv(m, 16, 256, 5, 0, outliers=3)
+    host.append(0, 0, k, v)
+    dev.append(0, 0, torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda())
+    q = oracle.normal(n * 64 * 256, 5, 3).reshape(n, 64, 256)
+    out, _ = dev.prefill_chunk(0, pos0, torch.from_numpy(q).cuda())
+    torch.cuda.synchronize()
+    rows = sorted({0, 1, 5, n // 2, n - 1})
+    want = [host.decode(0, pos0 + i + 1, q[i], nthreads=8)[0] for i in rows]
+    assert max(oracle.rel_err(out[i].cpu().numpy(), w) for i, w in zip(rows, want)) <= 1e-4

@@ -205,12 +205,13 @@ static int choose_path(const DecodePlan &p) {
   return kPathSplit;
 }
 
-// Contexts a decode takes in one workgroup per KV group (bkv_short.hip): six V tiles with q8_0 V, seven (pages,
-// which cost it a lookup per load) or eight with fp16 V. us of one layer of 8 against the stream kernel, q8_0:
-// 6.0 / 17.1 at 64 keys, 13.2 / 17.1 at 300, 16.8 / 17.2 at 385, 17.7 / 17.2 at 447 (8 KV heads 17.2 / 17.0 at 385);
-// against the resident kernel, fp16 V: 9.1 / 23.3 at 64, 14.2 / 22.4 at 256, 21.9 / 22.5 at 511.
-static int short_decode_keys(int vfmt, bool paged) {
-  if (vfmt == BKV_Q8_0) return 384;
+// Contexts a decode takes in one workgroup per KV group (bkv_short.hip): six V tiles with q8_0 V (seven with q8_0
+// K, no pages and up to 4 KV heads), seven (pages, which cost it a lookup per load) or eight with fp16 V. us of
+// one layer of 8 against the stream kernel, q8_0: 6.2 / 17.1 at 64 keys, 12.8 / 17.1 at 300, 16.5 / 17.1 at 400,
+// 17.2 / 17.1 at 440 (8 KV heads 17.0 / 17.0 at 385, 17.5 / 17.0 at 420); with fp16 K 15.0 / 18.6 at 300; against
+// the resident kernel, fp16 V: 14.9 / 22.0 at 300, 20.3 / 21.9 at 500.
+static int short_decode_keys(int kfmt, int vfmt, bool paged, int nkv) {
+  if (vfmt == BKV_Q8_0) return kfmt == BKV_Q8_0 && !paged && nkv <= 4 ? 448 : 384;
   return paged ? 448 : kShortKeys;
 }
 
@@ -308,7 +309,7 @@ static int decode_common(const bkv_cache_desc *d, int layer, uint32_t nfill, con
   L.base = kstart;
 
   const int path = choose_path(p);
-  if (forced_path() < 0 && path != kPathSplit && nfill <= (uint32_t)short_decode_keys(d->v_fmt, d->page_tokens > 0)) {
+  if (forced_path() < 0 && path != kPathSplit && nfill <= (uint32_t)short_decode_keys(d->k_fmt, d->v_fmt, d->page_tokens > 0, d->nkv)) {
     // the single launch of a short context: one workgroup per KV group
     ShortArgs sa{};
     sa.L = L; sa.nkv = d->nkv; sa.nh = d->nh; sa.pos0 = nfill - 1; sa.n_q = 1; sa.scale = d->scale;

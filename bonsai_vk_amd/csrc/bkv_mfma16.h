@@ -61,8 +61,8 @@ __device__ __forceinline__ void split_prod(h2 b, h2 s, h2 &hi, h2 &lo) {
 //    NaN: p = 0 does not take them out, as 0 * Inf is NaN. The rows of one query at a time are computed with
 //    the keys past that query's last one zeroed in the V operand, and the other rows' results dropped.
 // A tile of either kind costs up to 2 x 4 times the MFMAs; ordinary values never have one. (us, with ordinary
-// scales and with every scale past 512: a decode of 300 keys 13.2 / 19.1, 6 queries onto 300 keys 16.8 / 26.5,
-// 6 onto 3000 47.2 / 59.0, 512 onto 8192 333 / 430.)
+// scales and with every scale past 512: a decode of 300 keys 12.8 / 19.0, 6 queries onto 300 keys 16.6 / 26.9,
+// 6 onto 3000 44.1 / 58.8, 512 onto 8192 333 / 430.)
 
 // bits 14 and 30: the low and high fp16 of w is 512 or more in magnitude, Inf or NaN
 __device__ __forceinline__ uint32_t scale_big(uint32_t w) { return w & (w << 1) & 0x40004000u; }

@@ -7,11 +7,11 @@
 // e in key order (the reference's serial fp32 sum, attn_vk.h:175-189), p16 = f16(e / sum) goes to LDS and
 // the PV runs on the matrix cores from V tiles that direct-to-LDS loads brought in behind the scores.
 // What bounds it: a chain of latencies (K rows, scores, exps, the serial sum at about 5 ns per key, V
-// tiles); past 384 keys with q8_0 V (448 with fp16 V and pages) a decode is faster where the stream or
-// resident kernel spreads the keys wider (short_decode_keys). Chunks take it to kShortKeys.
+// tiles); past 384 to 448 keys (512 with contiguous fp16 V) a decode is faster where the stream or resident
+// kernel spreads the keys wider (short_decode_keys). Chunks take it to kShortKeys (short_chunk).
 // Scores, e, sums and p16 are bit-identical to the other kernels'; the PV sum's order differs. Its error
-// given p16 (2-norm, q8_0 V) is 6.6e-8 at 64 keys, 8.3e-8 at 300, 8.8e-8 at 384 (the stream kernel's 6.9e-8,
-// 8.5e-8, 8.4e-8; one fp32 chain over all products 8.8e-8, 1.7e-7, 1.9e-7).
+// given p16 (2-norm, q8_0 V) is 6.6e-8 at 64 keys, 7.7e-8 at 300, 8.5e-8 at 440 (the stream kernel's 6.9e-8,
+// 8.5e-8, 8.6e-8; one fp32 chain over all products 8.8e-8, 1.7e-7, 2.0e-7).
 #include <type_traits>
 
 #include "bkv_device.h"
@@ -497,8 +497,9 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
     }
   };
   // Chains per value by tile (mod NS) and key half, and the small parts of q8_0 products on their own: the
-  // matrix cores round every step of a chain down (see the header).
-  constexpr int NS = NR == 4 ? 2 : 3;
+  // matrix cores round every step of a chain down (see the header). (The loop takes NS tiles a turn: chosen by a
+  // branch at the end of a tile instead, a decode of 300 keys takes 13.2 to 14.0 us, not 12.8.)
+  constexpr int NS = 3;
   f4 zh[NS][2][2] = {}, zl[2][1] = {};             // [tile mod NS][key half][mt]; [mt]
   auto careful = [&](int t) {
     f4 z[2][1] = {{zh[0][0][0]}, {zh[0][0][1]}};
@@ -519,93 +520,86 @@ __global__ __launch_bounds__(kShNT, 1) void short_kernel(ShortArgs a) {
     zh[0][0][1] = z[1][0];
   };
   unsigned later = 0;                              // fp16 V: tiles that need pv_tile_careful (of this wave's dims)
-  // (CAREFUL: q8_0 V with a scale past the plain products, a loop of its own so that the other stays small)
-  auto loop = [&](auto mode) {
-    constexpr bool CAREFUL = decltype(mode)::value;
-    for (int t = 0; t < nt; ++t) {
-      // Tile t + NB - 1 goes into tile t - 1's buffer once every wave has read that one; later tiles are waited
-      // for in order, the younger ones' loads left in flight.
-      if (t > 0 && nt > NB) {
-        if (t >= NB) {
-          if (t + 1 >= nt) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ND) : "memory");
-        }
-        lds_barrier();
-        if (t + NB - 1 < nt) dma_tile(t + NB - 1);
+  // Tile t's values in its buffer: tile t + NB - 1 goes into tile t - 1's buffer once every wave has read that
+  // one; later tiles are waited for in order, the younger ones' loads left in flight.
+  auto arrive = [&](int t) {
+    if (t > 0 && nt > NB) {
+      if (t >= NB) {
+        if (t + 1 >= nt) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ND) : "memory");
       }
-      char *vt = s_v[t % NB];
-      if (append && t == nt - 1) {                 // the appended row, this wave's dims, over its loaded copy
-        const int r = (kend - 1) & 63;
+      lds_barrier();
+      if (t + NB - 1 < nt) dma_tile(t + NB - 1);
+    }
+    char *vt = s_v[t % NB];
+    if (append && t == nt - 1) {                   // the appended row, this wave's dims, over its loaded copy
+      const int r = (kend - 1) & 63;
+      if constexpr (VF) {
+        const int i = r >> 2;
+        if (lane < 2)
+          *reinterpret_cast<uint4 *>(vt + 1024 * i + 64 * ((2 * w + lane) ^ (i & 3)) + 16 * (r & 3)) = s_row[1][2 * w + lane];
+      } else {                                     // (and over the padding's copies: see the scales)
+        const int c = 4 * (w & 3) + (lane & 3);
+        for (int rr = r + (lane >> 2); rr < 64; rr += 16) {
+          const int i = rr >> 2;
+          *reinterpret_cast<uint4 *>(vt + 1024 * (i + 16 * (w >> 2)) + 64 * (c ^ (2 * ((i >> 1) & 3))) + 16 * (rr & 3)) =
+              s_row[1][4 * w + (lane & 3)];
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  };
+  auto tile = [&](int t, f4 (&zp)[2][2]) {
+    arrive(t);
+    uint32_t x[2][2][4], s[2][4];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) ops(t, ks, mt, x[ks][mt], s[ks]);
+    if (!VF && 64 * t + 63 > lim0) {               // some rows do not see some of the tile's keys
+      uint32_t nf = 0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) nf |= non_finite(x[i >> 3][(i >> 2) & 1][i & 3]);
+      if (__any(nf != 0u)) {
+        later |= 1u << t;
+        return;
+      }
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const h8 bp = rows(t, ks);
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) {
+        const uint32_t (&xk)[4] = x[ks][mt];
         if constexpr (VF) {
-          const int i = r >> 2;
-          if (lane < 2)
-            *reinterpret_cast<uint4 *>(vt + 1024 * i + 64 * ((2 * w + lane) ^ (i & 3)) + 16 * (r & 3)) = s_row[1][2 * w + lane];
-        } else {                                   // (and over the padding's copies: see the scales)
-          const int c = 4 * (w & 3) + (lane & 3);
-          for (int rr = r + (lane >> 2); rr < 64; rr += 16) {
-            const int i = rr >> 2;
-            *reinterpret_cast<uint4 *>(vt + 1024 * (i + 16 * (w >> 2)) + 64 * (c ^ (2 * ((i >> 1) & 3))) + 16 * (rr & 3)) =
-                s_row[1][4 * w + (lane & 3)];
+          uint32_t hw[4], lw[4];
+#pragma unroll
+          for (int pp = 0; pp < 4; ++pp) {
+            h2 hi, lo;
+            split_prod(as_h2(xk[pp]), as_h2(s[ks][pp]), hi, lo);
+            hw[pp] = as_u(hi);
+            lw[pp] = as_u(lo);
           }
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      }
-      if constexpr (CAREFUL) {
-        careful(t);
-      } else {
-        uint32_t x[2][2][4], s[2][4];
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-          for (int mt = 0; mt < 2; ++mt) ops(t, ks, mt, x[ks][mt], s[ks]);
-        const h8 bp[2] = {rows(t, 0), rows(t, 1)};
-        bool plain = true;
-        if (!VF && 64 * t + 63 > lim0) {           // some rows do not see some of the tile's keys
-          uint32_t nf = 0;
-#pragma unroll
-          for (int i = 0; i < 16; ++i) nf |= non_finite(x[i >> 3][(i >> 2) & 1][i & 3]);
-          plain = !__any(nf != 0u);
-          if (!plain) later |= 1u << t;
-        }
-        if (plain) {
-          h8 hi[2][2];
-#pragma unroll
-          for (int mt = 0; mt < 2; ++mt) {
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-              const uint32_t (&xk)[4] = x[ks][mt];
-              if constexpr (VF) {
-                uint32_t hw[4], lw[4];
-#pragma unroll
-                for (int pp = 0; pp < 4; ++pp) {
-                  h2 h, l;
-                  split_prod(as_h2(xk[pp]), as_h2(s[ks][pp]), h, l);
-                  hw[pp] = as_u(h);
-                  lw[pp] = as_u(l);
-                }
-                hi[ks][mt] = __builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3]));
-                zl[mt][0] = mfma16(__builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3])), bp[ks], zl[mt][0]);
-              } else {
-                hi[ks][mt] = __builtin_bit_cast(h8, make_uint4(xk[0], xk[1], xk[2], xk[3]));
-              }
-            }
-          }
-          auto step = [&](f4 (&zp)[2][2]) {
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-              for (int mt = 0; mt < 2; ++mt) zp[ks][mt] = mfma16(hi[ks][mt], bp[ks], zp[ks][mt]);
-          };
-          const int ts = t % NS;
-          if (ts == 0) step(zh[0]);
-          else if (ts == 1) step(zh[1]);
-          else step(zh[NS - 1]);
+          zp[ks][mt] = mfma16(__builtin_bit_cast(h8, make_uint4(hw[0], hw[1], hw[2], hw[3])), bp, zp[ks][mt]);
+          zl[mt][0] = mfma16(__builtin_bit_cast(h8, make_uint4(lw[0], lw[1], lw[2], lw[3])), bp, zl[mt][0]);
+        } else {
+          zp[ks][mt] = mfma16(__builtin_bit_cast(h8, make_uint4(xk[0], xk[1], xk[2], xk[3])), bp, zp[ks][mt]);
         }
       }
     }
   };
-  if (__builtin_expect(VF && s_big != 0u, 0)) loop(std::integral_constant<bool, VF != 0>{});
-  else loop(std::false_type{});
+  if (__builtin_expect(VF && s_big != 0u, 0)) {    // a scale past the plain products: a loop of its own
+    for (int t = 0; t < nt; ++t) {
+      arrive(t);
+      careful(t);
+    }
+  } else {
+    for (int t = 0; t < nt; t += NS) {
+      tile(t, zh[0]);
+      if (t + 1 < nt) tile(t + 1, zh[1]);
+      if (NS == 3 && t + 2 < nt) tile(t + 2, zh[NS - 1]);
+    }
+  }
   if constexpr (!VF)                               // (the last two tiles at most, still in their buffers)
     for (int t = 0; later != 0u; ++t, later >>= 1)
       if (later & 1u) careful(t);

@@ -499,12 +499,14 @@ int bkv_decode_step_qg(const bkv_cache_desc *d, int layer, uint32_t pos, const f
                             workspace, ws_bytes, stream, 2 * kHd, 2 * kHd);
 }
 
-// Whether a chunk of 2 to kPxMinQ - 1 queries runs as one chunk (true) or as decode rows: the chunk takes
-// about 26 us and 6.2 ns per key of its last row (its serial sums) whatever its length, a decode row 17 us
-// and 0.4 ns per key. us for the attention, rows / chunk: 2 queries at 3000 keys 37 / 47, 3 at 3000 55 / 47,
-// 6 at 3000 110 / 49, 3 at 8000 61 / 73, 8 at 8000 160 / 73, 6 at 32000 168 / 228, 12 at 32000 335 / 212.
+// Whether a chunk of two or more queries runs as one chunk (true; always from kPxMinQ on) or as decode rows:
+// the chunk takes about 24 us and 6.2 ns per key of its last row (its serial sums) whatever its length, a decode
+// row 17 us and 0.4 ns per key. us for the attention, rows / chunk, q8_0: 3 queries at 3000 keys 55 / 42, 6 at 3000
+// 110 / 44, 6 at 8000 119 / 74, 3 at 8000 61 / 73, 8 at 8000 160 / 73, 6 at 32000 168 / 228, 12 at 32000 335 / 212;
+// fp16: 6 at 8000 167 / 75. Over every format pair, 64-token pages, 1 to 16 KV heads, 520 to 64000 keys and 2 to 15
+// queries (1216 combinations) the choice is nowhere behind the rows.
 static bool px_worthwhile(int n_q, int64_t keys) {
-  return n_q >= kPxMinQ || (n_q > 1 && n_q * (170000 + 4 * keys) > 260000 + 62 * keys);
+  return n_q >= kPxMinQ || n_q * (170000 + 4 * keys) > 260000 + 62 * keys;
 }
 
 // Whether a chunk of a short context runs in the short kernel, whose workgroups (4 queries of a KV group) fill
@@ -533,7 +535,9 @@ static int prefill_common(const bkv_cache_desc *d, int layer, uint32_t pos0, int
   if (!workspace) return BKV_EWORKSPACE;
   if (((uintptr_t)workspace & 255u) != 0) return BKV_EALIGN;
   const size_t base = prefill_base(d);
-  if (!prefill_mfma_requested() && n_q > 1 && (int64_t)pos0 + n_q <= kShortKeys && short_chunk(d->nkv, pos0, n_q)) {
+  // (a forced decode path also decides how the rows of a chunk below kPxMinQ queries run)
+  const bool rows = n_q == 1 || (n_q < kPxMinQ && forced_path() >= 0);
+  if (!prefill_mfma_requested() && !rows && (int64_t)pos0 + n_q <= kShortKeys && short_chunk(d->nkv, pos0, n_q)) {
     // a short context: one launch, 4 queries per workgroup (the workspace is asked for all the same, so
     // that a caller meets its size at the first chunk and not at a later one)
     const size_t need = n_q >= kPxMinQ ? px_layout(d->nh, d->nkv, (int64_t)pos0 + n_q, kPxSlice, base).total
@@ -544,7 +548,7 @@ static int prefill_common(const bkv_cache_desc *d, int layer, uint32_t pos0, int
     a.q = q; a.qs = qs; a.gate = gate; a.gs = gs; a.out = out; a.out_gated = out_gated;
     return hip_fail(launch_short(a, d->k_fmt, d->v_fmt, stream));
   }
-  if (!prefill_mfma_requested() && px_worthwhile(n_q, (int64_t)pos0 + n_q) &&
+  if (!prefill_mfma_requested() && !rows && px_worthwhile(n_q, (int64_t)pos0 + n_q) &&
       (n_q >= kPxMinQ || ws_bytes >= px_layout(d->nh, d->nkv, (int64_t)pos0 + n_q, kPxSlice, base).total)) {
     // the exact kernels, in equal slices (of kPxSlice queries in a workspace without room for more)
     const int64_t ctx = (int64_t)pos0 + n_q;

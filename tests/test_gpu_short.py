@@ -138,3 +138,19 @@ def test_short_chunk_of_many_kv_heads(kf, vf, pos0, n):
     rows = sorted({0, 1, 5, n // 2, n - 1})
     want = [host.decode(0, pos0 + i + 1, q[i], nthreads=8)[0] for i in rows]
     assert max(oracle.rel_err(out[i].cpu().numpy(), w) for i, w in zip(rows, want)) <= 1e-4
+
+
+@pytest.mark.parametrize("forced", ["split", "resident", "stream"])
+@pytest.mark.parametrize("pos0,n", [(100, 3), (700, 5)])
+def test_forced_path_in_small_chunks(pos0, n, forced, monkeypatch):
+    """BKV_DECODE decides how the rows of a chunk of 2 to 15 queries run: each equals the forced decode."""
+    say(f"forced {forced}: chunk of {n} onto {pos0}")
+    monkeypatch.setenv("BKV_DECODE", forced)
+    c, _, k, v = caches(pos0 + n, BKV_Q8_0, BKV_Q8_0, 0)
+    c.append(0, pos0 + n - 1, k[-1:], v[-1:])
+    q = queries(n, "normal")
+    out, _ = c.prefill_chunk(0, pos0, q)
+    for i in range(n):
+        want, _ = c.decode(0, pos0 + i + 1, q[i].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(out[i], want), i

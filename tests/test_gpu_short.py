@@ -2,12 +2,13 @@
 resident and chunk kernels, which the other tests hold to the oracle: scores' e, sums and cache bytes bit
 for bit, outputs to the fp32 order of the PV sum (each a sum of at most 512 exact products of magnitude
 below the row's largest |v|: 512 * 2^-24 of it bounds the difference of two orders)."""
+import numpy as np
 import pytest
 import torch
 
 import oracle
 from bonsai_vk_amd import BKV_F16, BKV_Q8_0, KvCache
-from tests.gpu_util import say
+from tests.gpu_util import pair, qg, say
 
 pytestmark = pytest.mark.gpu
 FMTS = [(BKV_Q8_0, BKV_Q8_0), (BKV_F16, BKV_F16), (BKV_F16, BKV_Q8_0), (BKV_Q8_0, BKV_F16)]
@@ -154,3 +155,63 @@ def test_forced_path_in_small_chunks(pos0, n, forced, monkeypatch):
         want, _ = c.decode(0, pos0 + i + 1, q[i].contiguous())
         torch.cuda.synchronize()
         assert torch.equal(out[i], want), i
+
+
+SYNC = slice(200 * 1024, 212 * 1024)               # of the workspace: the sync lines of the exchanging kernels
+
+
+def limit(kf, vf, page):
+    """the longest decode the short kernel takes at 4 KV heads"""
+    if vf == BKV_Q8_0:
+        return 448 if kf == BKV_Q8_0 and not page else 384
+    return 448 if page else 512
+
+
+@pytest.mark.parametrize("kf,vf", FMTS)
+@pytest.mark.parametrize("page", [0, 3, 64])
+def test_short_decode_against_the_oracle(kf, vf, page, monkeypatch):
+    """Unforced decodes on either side of every limit and tile: which kernel ran (the exchanging ones advance their
+    generation words in the workspace, the short one leaves them), e, the serial sums and p16 bit for bit the
+    oracle's, cache bytes, output; a window; at the limit also appended into slots of NaN bytes."""
+    monkeypatch.setenv("BKV_KEEP_INTERMEDIATES", "1")
+    say(f"short decode against the oracle kf={kf} vf={vf} page={page}")
+    m, kw = 520, {}
+    cap = m
+    if page:
+        pool = -(-m // page) + 2
+        kw = dict(page_tokens=page, max_pages=pool, block_table=np.random.default_rng(page).permutation(pool)[None].astype(np.int32))
+        cap = pool * page
+    dev, host = pair(1, cap, kf, vf, **kw)
+    for t in (dev.k_data, dev.k_scales, dev.v_data, dev.v_scales):
+        if t is not None:
+            t.fill_(255)
+    k, v = oracle.synth_kv(m, 4, 256, 17, 0, outliers=3)
+    q, g = qg(17, 0)
+    qd, gd = torch.from_numpy(q).cuda(), torch.from_numpy(g).cuda()
+    done = 0
+    for n in (1, 17, 64, 65, 129, 256, 257, 320, 321, 384, 385, 447, 448, 449, 511, 512, 513):
+        host.append(0, done, k[done:n], v[done:n])
+        if n - 1 > done:
+            dev.append(0, done, torch.from_numpy(k[done:n - 1]).cuda(), torch.from_numpy(v[done:n - 1]).cuda())
+        done = n
+        before = dev.workspace[SYNC].clone()
+        out, og = dev.decode_step(0, n - 1, torch.from_numpy(k[n - 1:n]).cuda(), torch.from_numpy(v[n - 1:n]).cuda(), qd, gd)
+        torch.cuda.synchronize()
+        assert torch.equal(before, dev.workspace[SYNC]) == (n <= limit(kf, vf, page)), n
+        want, wg, sc, pr, p16 = host.decode(0, n, q, g, nthreads=8, debug=True)
+        _, e, s, st = dev.debug_intermediates(n)
+        x = sc * np.float32(0.0625)
+        assert oracle.bit_diff(e.numpy(), np.exp((x - x.max(axis=1, keepdims=True)).astype(np.float64)).astype(np.float32)) == 0, n
+        p = (e.numpy() / s.numpy()[:, None]).astype(np.float32)
+        assert oracle.bit_diff(p, pr) == 0 and np.array_equal(oracle.f32_to_f16(p), p16) and int(st.abs().sum()) == 0, n
+        assert oracle.rel_err(out.cpu().numpy(), want) <= 1e-4 and oracle.rel_err(og.cpu().numpy(), wg) <= 1e-4, n
+    for a, b in zip(dev.host_arrays(), host.arrays()):
+        if b is not None:                          # (the slots after the last token still hold what they did)
+            slots = [host.slot(0, i) for i in range(done)]
+            assert np.array_equal(a.numpy()[0, slots], b[0, slots])
+    _, win = pair(1, 400, kf, vf)
+    win.append(0, 0, k[113:513], v[113:513])
+    wlen = min(limit(kf, vf, page) - 70, 400)
+    out, _ = dev.decode_window(0, 113, 113 + wlen, qd)
+    torch.cuda.synchronize()
+    assert oracle.rel_err(out.cpu().numpy(), win.decode(0, wlen, q)[0]) <= 1e-4

@@ -464,9 +464,11 @@ hipError_t launch_prefill(const PrefillArgs &a, int kf, int vf, hipStream_t st) 
 //           them in key order (the reference's serial fp32 sum, attn_vk.h:175-189).
 //   pv      p16 = f16(e / sum) (the correctly rounded fp32 quotient, from e * (1/sum) by two remainder
 //           corrections, then round to nearest even), and sum p16 * v on the matrix cores for 128
-//           rows and one of pv_split key ranges.
-//   merge   the key ranges' partials added in order, and the gate.
-// Only the PV sum runs in another order than the reference (fp32 accumulation of exact products).
+//           rows (slices of up to 16 queries: 64) and one of pv_split key ranges. Tiles whose V is past
+//           the plain products, or not finite where a row does not see the key, take pv_tile_careful.
+//   merge   the key ranges' partials added by eights, the eights in fp64, and the gate.
+// Only the PV sum runs in another order than the reference (fp32 accumulation of exact products; slices
+// of up to 16 queries add their tiles in fp64).
 
 // scratch accesses (plain loads and stores: the scratch round trips are served largely by the
 // memory-side cache, which non-temporal accesses bypass)

@@ -7,7 +7,7 @@
 // e in key order (the reference's serial fp32 sum, attn_vk.h:175-189), p16 = f16(e / sum) goes to LDS and
 // the PV runs on the matrix cores from V tiles that direct-to-LDS loads brought in behind the scores.
 // What bounds it: a chain of latencies (K rows, scores, exps, the serial sum at about 5 ns per key, V
-// tiles); past 384 to 448 keys (512 with contiguous fp16 V) a decode is faster where the stream or resident
+// tiles); past 384, 448 or 512 keys, by format and layout, a decode is faster where the stream or resident
 // kernel spreads the keys wider (short_decode_keys). Chunks take it to kShortKeys (short_chunk).
 // Scores, e, sums and p16 are bit-identical to the other kernels'; the PV sum's order differs. Its error
 // given p16 (2-norm, q8_0 V) is 6.6e-8 at 64 keys, 7.7e-8 at 300, 8.5e-8 at 440 (the stream kernel's 6.9e-8,
